@@ -9,7 +9,7 @@
 //   qr fp32, kc/vc     q/k RMSNorm (optional) + RoPE with the model's inverse frequencies, k and v
 //                      appended to the per-layer fp32 KV cache at pos0 .. pos0 + T - 1 (k_qk_rope)
 //   ob [T, nh*hd] fp16 causal softmax attention over the cache, grouped-query, optional sigmoid gate
-//                      (k_attention)
+//                      (hq_attention.hip)
 //   x += hq_gemm(o, ob)                               (accumulate into the residual)
 //   hb = RMSNorm(x) fp16
 //   fb = silu(gate . hb) * (up . hb) fp16: where gate and up share a block type and shape they are
@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "hq.h"
+#include "hq_attention.h"
 #include "hq_backend.h"
 #include "hq_device.h"
 #include "hq_internal.h"
@@ -97,11 +98,6 @@ DEV void deq8(const hq_dev_mat &W, size_t r, int g, float (&w)[8]) {
 DEV float wave_sum(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-DEV float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
     return v;
 }
 
@@ -183,60 +179,6 @@ __global__ void __launch_bounds__(64) k_qk_rope(const float *__restrict__ qb, co
     }
 }
 
-// One wave per (token t, query head j): causal softmax attention of query pos0 + t over cache
-// positions 0 .. pos0 + t of kv head j / (nh / nkv), online over chunks of 64 positions (lane s
-// scores position s0 + s); output fp16 [T, nh * hd], times sigmoid(gate) when gated
-// (src/cpu_backend.c:103-131).
-__global__ void __launch_bounds__(64) k_attention(const float *__restrict__ qr, const float *__restrict__ qb,
-                                                  const float *__restrict__ kc, const float *__restrict__ vc,
-                                                  _Float16 *__restrict__ out, int nh, int nkv, int hd, int qw,
-                                                  int gated, int pos0, float scale) {
-    __shared__ float qs[256];
-    const int t = blockIdx.x, j = blockIdx.y, lane = threadIdx.x, kvw = nkv * hd, g = j / (nh / nkv);
-    const int n = pos0 + t + 1;
-    for (int d = lane; d < hd; d += 64) qs[d] = qr[((size_t)t * nh + j) * hd + d];
-    __syncthreads();
-    float m = -INFINITY, l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
-    const float *kh = kc + (size_t)g * hd, *vh = vc + (size_t)g * hd;
-    for (int s0 = 0; s0 < n; s0 += 64) {
-        const int s = s0 + lane;
-        float sc = -INFINITY;
-        if (s < n) {
-            const float *kr = kh + (size_t)s * kvw;
-            float acc = 0.f;
-            for (int d = 0; d < hd; d += 4) {
-                const float4 k4 = *(const float4 *)(kr + d);
-                acc += qs[d] * k4.x + qs[d + 1] * k4.y + qs[d + 2] * k4.z + qs[d + 3] * k4.w;
-            }
-            sc = acc * scale;
-        }
-        const float mn = fmaxf(m, wave_max(sc));
-        const float pr = s < n ? expf(sc - mn) : 0.f;
-        const float alpha = expf(m - mn);  // 0 before the first chunk (m = -inf)
-        l = l * alpha + wave_sum(pr);
-#pragma unroll
-        for (int i = 0; i < 4; i++) o[i] *= alpha;
-        const int cnt = n - s0 < 64 ? n - s0 : 64;
-        for (int e = 0; e < cnt; e++) {
-            const float pe = __shfl(pr, e, 64);
-            const float *vr = vh + (size_t)(s0 + e) * kvw;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (lane + 64 * i < hd) o[i] += pe * vr[lane + 64 * i];
-        }
-        m = mn;
-    }
-    const float *gate = qb + (size_t)t * qw + (size_t)j * hd * 2 + hd;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int d = lane + 64 * i;
-        if (d >= hd) continue;
-        float y = o[i] / l;
-        if (gated) y *= 1.0f / (1.0f + expf(-gate[d]));
-        out[((size_t)t * nh + j) * hd + d] = (_Float16)y;
-    }
-}
-
 __global__ void __launch_bounds__(256) k_swiglu(const float *__restrict__ g, const float *__restrict__ u,
                                                 _Float16 *__restrict__ out, size_t n) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
@@ -315,6 +257,9 @@ struct HipBackend {
     _Float16 *hb = nullptr, *ob = nullptr, *fb = nullptr;
     uint32_t *d_tok = nullptr, *d_ids = nullptr;
     float *d_logits = nullptr, *d_hidden = nullptr;
+    float *att_part = nullptr;  // partial rows of the attention's split blocks, and their counters
+    int *att_cnt = nullptr;
+    int n_cu = 0;
     int chunk = CHUNK, last_T = 0;
     size_t snap_pos = 0;
     bool has_snap = false;
@@ -406,8 +351,8 @@ int run_layers(HipBackend *b, int T, int pos0) {
                                                     L.kc, L.vc, nh, nkv, hd, (int)c.rot_dim, qw, c.attn_gate, pos0,
                                                     c.qk_norm);
         BCK(hipGetLastError());
-        k_attention<<<dim3(T, nh), 64, 0, st>>>(b->qr, b->qb, L.kc, L.vc, b->ob, nh, nkv, hd, qw, c.attn_gate, pos0, scale);
-        BCK(hipGetLastError());
+        const HqAttnArgs at = {b->qr, b->qb, L.kc, L.vc, b->ob, b->att_part, b->att_cnt, T, nh, nkv, hd, qw, c.attn_gate, pos0, scale};
+        BCK(hq_launch_attention(at, b->n_cu, st));
         if (gemm(b, L.o, b->ob, T, b->x, true)) return -1;
         k_rmsnorm<_Float16><<<T, 256, 0, st>>>(b->x, L.post_norm, off, eps, b->hb, H);
         BCK(hipGetLastError());
@@ -545,6 +490,11 @@ int init(HipBackend *b, const hq_ref_model_t *m, size_t max_seq) {
         dalloc(b, (void **)&b->d_tok, CH * 4) || dalloc(b, (void **)&b->d_ids, MAX_IDS * 4) ||
         dalloc(b, (void **)&b->d_logits, MAX_IDS * 4) || dalloc(b, (void **)&b->d_hidden, H * 4))
         return -1;
+    BCK(hipDeviceGetAttribute(&b->n_cu, hipDeviceAttributeMultiprocessorCount, b->device));
+    if (dalloc(b, (void **)&b->att_part, hq_attn_work_bytes((int)hd, b->n_cu)) ||
+        dalloc(b, (void **)&b->att_cnt, HQ_ATTN_MAX_BLOCKS * sizeof(int)))
+        return -1;
+    BCK(hipMemset(b->att_cnt, 0, HQ_ATTN_MAX_BLOCKS * sizeof(int)));
     // every projection must take its input width and give the next one's
     for (uint32_t l = 0; l < c.n_layers; l++) {
         const DevLayer &d = b->L[l];

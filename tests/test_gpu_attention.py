@@ -1,0 +1,41 @@
+"""The backend's attention (hq_attention.hip) at the edges of its tiles: head sizes around the 64-wide
+padding, grouped heads, row counts around 16 and 32, one and several position ranges per row block,
+against the oracle's CPU forward of the same one-layer model.
+
+The tolerance is the logits' bar of every forward test: GEMM operands are rounded to fp16 (2^-11 each,
+logits of size ~1), attention itself is fp32 on both sides.
+"""
+import numpy as np
+import pytest
+
+import synth
+from conftest import max_abs
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # heads, kv heads, head_dim, prefix, tokens
+    (8, 8, 64, 0, 1), (8, 8, 64, 0, 31), (8, 8, 64, 0, 33), (8, 2, 64, 0, 129), (4, 1, 64, 500, 1), (8, 8, 64, 300, 17),
+    (8, 4, 40, 0, 70), (4, 4, 96, 33, 20), (8, 2, 128, 0, 130), (16, 4, 128, 257, 3), (2, 1, 160, 0, 67), (2, 2, 192, 40, 9),
+    (2, 1, 256, 0, 50), (4, 2, 256, 190, 1), (40, 8, 64, 0, 270), (48, 16, 128, 0, 250),
+]
+
+
+@pytest.mark.parametrize("nh,nkv,hd,prefix,T", CASES)
+def test_attention_edges(hqlib, oracle, nh, nkv, hd, prefix, T):
+    cfg = dict(synth.TINY_LLAMA, n_layers=1, hidden=256, intermediate=256, vocab=512, n_heads=nh, n_kv_heads=nkv, head_dim=hd,
+               rot_dim=hd)
+    model = synth.tiny_llama(nh + hd + T, cfg)
+    tokens, ids = synth.tiny_llama_prompt(7, T=prefix + T, vocab=512, n_ids=16)
+    be = hqlib.HipBackend(hqlib.RefModelView(model), prefix + T)
+    if prefix:
+        be.forward(tokens[:prefix])
+    got = be.forward(tokens[prefix:], ids)
+    again = None
+    if prefix:  # the same rows as part of one longer pass
+        be.reset()
+        again = be.forward(tokens, ids)
+    be.destroy()
+    ref = oracle.llama_forward(model, tokens, ids)
+    print(f"[gpu] attention {nh}/{nkv} x {hd}, {prefix} + {T}: max_abs {max_abs(got, ref):.2e}", flush=True)
+    assert max_abs(got, ref) <= 1e-2
+    assert again is None or max_abs(again, got) <= 1e-3
