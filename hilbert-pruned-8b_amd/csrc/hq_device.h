@@ -315,7 +315,6 @@ DEV void store8_out(void *C, int N, int m, int n, f4 v0, f4 v1, bool wide, int c
 template <int BM, int BN, int NT, int MAXP, class Args>
 DEV void tile_finish(const char *lds, const Args &g, int m0, int n0, int tile, int part, int *flag) {
     constexpr int LD = BN + 4, CH = BN / 8, NCH = BM * CH, CPT = (NCH + NT - 1) / NT;  // 8-value chunks
-    static_assert(NCH % NT == 0 || NCH < NT, "chunks per thread");
     constexpr uint32_t TILE = BM * BN * 4;  // bytes per partial tile
     const int M = g.M, N = g.N;
     const bool wide = (N & 7) == 0 && ((uintptr_t)g.C & 15u) == 0;
