@@ -365,6 +365,25 @@ extern "C" int hq_mat_upload_pair(const hq_wmat_t *gate, const hq_wmat_t *up, in
     return 0;
 }
 
+extern "C" int hq_internal_upload_cat(const hq_wmat_t *const *w, int n, int device, hq_mat **out) {
+    *out = nullptr;
+    size_t rb = 0;
+    uint64_t rows = 0;
+    for (int i = 0; i < n; i++) {
+        if (check_wmat(w[i], "hq_mat_upload", &rb)) return -1;
+        if (w[i]->ggml_type != w[0]->ggml_type || w[i]->cols != w[0]->cols)
+            return fail("hq_mat_upload: matrices of different types or widths cannot be one");
+        rows += w[i]->rows;
+    }
+    if (rows > (1u << 30)) return fail("hq_mat_upload: %llu rows too many", (unsigned long long)rows);
+    auto row_ptr = [&](uint32_t r) {
+        int i = 0;
+        while (r >= w[i]->rows) r -= w[i++]->rows;
+        return (const uint8_t *)w[i]->data + (size_t)storage_row(w[i]->rows, w[i]->perm_heads, r) * rb;
+    };
+    return upload_rows(w[0]->ggml_type, (uint32_t)rows, w[0]->cols, row_ptr, device, "hq_mat_upload", out);
+}
+
 extern "C" void hq_mat_free(hq_mat *m) {
     if (!m) return;
     if (use_device(m->device) == 0) (void)hipFree(m->alloc);
@@ -684,7 +703,9 @@ extern "C" int hq_gemm_swiglu(const hq_mat *pair, const uint16_t *A, int M, uint
         uint16_t *Op = out + m0 * (N2 / 2);
         HqGemmWork wk = {};
         int fused = 0;
-        if (mc > 1) {
+        if (mc == 1) {
+            HIPCK(hq_launch_gemv_pair(&pair->m, Ap, Op, S(stream), &fused));
+        } else {
             if (gemm_work(pair, mc, stream, &wk)) return -1;
             HIPCK(hq_launch_gemm_swiglu(&pair->m, Ap, mc, Op, wk, S(stream), &fused));
         }

@@ -33,6 +33,9 @@ namespace {
 
 DEV f4 mfma4(float a, float b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
+typedef float f2 __attribute__((ext_vector_type(2)));
+constexpr int ATT_SPLITS = 64;  // most workgroups a row block's positions are split over
+
 struct Args {
     HqAttnArgs a;
     int rep, R, nblk, splits;
@@ -245,19 +248,34 @@ __global__ void __launch_bounds__(64 * W) k_attn(Args g) {
     }
     __syncthreads();
     if (!last) return;
+    // each split's (max, sum) per row once into LDS, then its sums four loads at a time
+    f2 *const ml = (f2 *)&os[0][0][0];
+    static_assert(ATT_SPLITS * ROWS * sizeof(f2) <= sizeof os, "the splits' maxima and sums in the waves' arena");
+    for (int x = threadIdx.x; x < g.splits * ROWS; x += 64 * W) {
+        const f4 v = buf_load16_sc1(rp, (uint32_t)(x * PARTF + HDP) * 4u, 0);
+        ml[x] = f2{v.x, v.y};
+    }
+    __syncthreads();
     for (int x = threadIdx.x; x < ROWS * (HDP / 4); x += 64 * W) {
         const int row = x / (HDP / 4), d = 4 * (x % (HDP / 4));
         if (row0 + row >= g.R) continue;
         float mm = -INFINITY;
-        for (int u = 0; u < g.splits; u++) mm = fmaxf(mm, buf_load16_sc1(rp, (uint32_t)((u * ROWS + row) * PARTF + HDP) * 4u, 0).x);
+        for (int u = 0; u < g.splits; u++) mm = fmaxf(mm, ml[u * ROWS + row].x);
         f4 v = zero;
         float lt = 0.f;
-        for (int u = 0; u < g.splits; u++) {
-            const uint32_t at = (uint32_t)((u * ROWS + row) * PARTF) * 4u;
-            const f4 ml = buf_load16_sc1(rp, at + HDP * 4u, 0), y = buf_load16_sc1(rp, at + (uint32_t)d * 4u, 0);
-            const float f = part_scale(ml.x, mm);
-            v += y * f;
-            lt += ml.y * f;
+        for (int u0 = 0; u0 < g.splits; u0 += 4) {
+            f4 y[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                y[e] = buf_load16_sc1(rp, (uint32_t)((std::min(u0 + e, g.splits - 1) * ROWS + row) * PARTF + d) * 4u, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (u0 + e < g.splits) {
+                    const f2 p = ml[(u0 + e) * ROWS + row];
+                    const float f = part_scale(p.x, mm);
+                    v += y[e] * f;
+                    lt += p.y * f;
+                }
         }
         finish(row, d, v, lt);
     }
@@ -293,7 +311,7 @@ hipError_t hq_launch_attention(const HqAttnArgs &a, int n_cu, hipStream_t st) {
     const int tiles = (a.pos0 + a.T + tp - 1) / tp;
     g.splits = 1;
     if (blocks < n_cu && blocks <= HQ_ATTN_MAX_BLOCKS)
-        g.splits = (int)std::max(1l, std::min((long)(n_cu / blocks), (long)((tiles + W - 1) / W)));
+        g.splits = (int)std::max(1l, std::min({(long)(n_cu / blocks), (long)((tiles + W - 1) / W), (long)ATT_SPLITS}));
     if (a.hd <= 64) {
         if (qb == 2) launch<64, 2, 32, 8>(g, st);
         else launch<64, 1, 32, 8>(g, st);

@@ -5,7 +5,8 @@
 // for LAYER_FULL layers), on the backend's stream:
 //   x [T, H] fp32      residual stream (embedding rows decoded from the GGUF blocks)
 //   hb [T, H] fp16     RMSNorm(x) * (off + w): the GEMM operand (k_rmsnorm_f16)
-//   q/k/v fp32         hq_gemm(q|k|v, hb)            (q rows interleave [q_h | gate_h] with the output gate)
+//   q/k/v fp32         hq_gemm(q|k|v, hb)            (q rows interleave [q_h | gate_h] with the output gate);
+//        of one block type they are resident as one matrix, and one hq_gemm fills rows [q | k | v]
 //   qr fp32, kc/vc     q/k RMSNorm (optional) + RoPE with the model's inverse frequencies, k and v
 //                      appended to the per-layer fp32 KV cache at pos0 .. pos0 + T - 1 (k_qk_rope)
 //   ob [T, nh*hd] fp16 causal softmax attention over the cache, grouped-query, optional sigmoid gate
@@ -14,8 +15,7 @@
 //   hb = RMSNorm(x) fp16
 //   fb = silu(gate . hb) * (up . hb) fp16: where gate and up share a block type and shape they are
 //        resident as one gate/up pair matrix (hq_mat_upload_pair) and fb comes from hq_gemm_swiglu
-//        (any T: the SwiGLU epilogue inside the GEMM's tiles for prefill shapes, the tuned GEMV over
-//        both halves at T = 1); otherwise (a Q4_K gate with a Q6_K up, as Q4_K_M files pair them)
+//        (any T: the SwiGLU epilogue inside the GEMM's or GEMV's kernel); otherwise (a Q4_K gate with a Q6_K up, as Q4_K_M files pair them)
 //        T = 1 runs k_gateup_swiglu (one pass over both matrices) and larger T two hq_gemm calls and
 //        k_swiglu
 //   x += hq_gemm(down, fb)
@@ -51,6 +51,11 @@ namespace {
 
 constexpr int CHUNK = 1024;    // tokens per layer-loop pass
 constexpr int MAX_IDS = 4096;  // readout ids per forward
+
+// Up to 64 tokens or readout ids as a kernel argument: a copy of them to the device costs a launch of its own.
+struct IdArgs {
+    uint32_t v[64];
+};
 
 // ------------------------------------------------------------------------------------ kernels
 // Eight consecutive weights 8g .. 8g + 7 of row r as fp32, bit-identical to the reference decoder
@@ -125,20 +130,21 @@ __global__ void __launch_bounds__(256) k_rmsnorm(const float *__restrict__ x, co
     for (int i = threadIdx.x; i < H; i += 256) out[(size_t)blockIdx.x * H + i] = (T)(xr[i] * inv * (off + w[i]));
 }
 
-// One wave per (token t, head j): heads j < nh are queries (q rows of qb, stride qw, [q | gate]
+// One wave per (token t, head j): heads j < nh are queries (q rows of qb, [q | gate]
 // per head when gated), the others keys of kv head j - nh (whose value row is copied alongside).
 // Optional q/k RMSNorm, then RoPE on the first rot dims (pairs i, i + rot/2) at position pos0 + t
 // (src/cpu_backend.c:86-102). Queries go to qr [T, nh, hd]; keys and values to the caches.
+// sq, sk, sv: row strides of qb, kb, vb.
 __global__ void __launch_bounds__(64) k_qk_rope(const float *__restrict__ qb, const float *__restrict__ kb,
                                                 const float *__restrict__ vb, const float *__restrict__ qn,
                                                 const float *__restrict__ kn, float off, float eps,
                                                 const float *__restrict__ inv_freq, float *__restrict__ qr,
                                                 float *__restrict__ kc, float *__restrict__ vc, int nh, int nkv, int hd,
-                                                int rot, int qw, int gated, int pos0, int qk_norm) {
+                                                int rot, int sq, int sk, int sv, int gated, int pos0, int qk_norm) {
     __shared__ float xs[256];
     const int t = blockIdx.x, j = blockIdx.y, lane = threadIdx.x, kvw = nkv * hd;
     const bool is_q = j < nh;
-    const float *src = is_q ? qb + (size_t)t * qw + (size_t)j * hd * (gated ? 2 : 1) : kb + (size_t)t * kvw + (size_t)(j - nh) * hd;
+    const float *src = is_q ? qb + (size_t)t * sq + (size_t)j * hd * (gated ? 2 : 1) : kb + (size_t)t * sk + (size_t)(j - nh) * hd;
     float *dst = is_q ? qr + ((size_t)t * nh + j) * hd : kc + (size_t)(pos0 + t) * kvw + (size_t)(j - nh) * hd;
     float v[4];
     float ss = 0.f;
@@ -175,7 +181,7 @@ __global__ void __launch_bounds__(64) k_qk_rope(const float *__restrict__ qb, co
             y = d < half ? xs[d] * cs - xs[d + half] * sn : xs[d] * cs + xs[d - half] * sn;
         }
         dst[d] = y;
-        if (!is_q) vc[(size_t)(pos0 + t) * kvw + (size_t)(j - nh) * hd + d] = vb[(size_t)t * kvw + (size_t)(j - nh) * hd + d];
+        if (!is_q) vc[(size_t)(pos0 + t) * kvw + (size_t)(j - nh) * hd + d] = vb[(size_t)t * sv + (size_t)(j - nh) * hd + d];
     }
 }
 
@@ -208,12 +214,23 @@ __global__ void __launch_bounds__(256) k_gateup_swiglu(hq_dev_mat Wg, hq_dev_mat
     if (lane == 0) out[i] = (_Float16)(silu(sg) * su);
 }
 
+// x[t] = embedding row of tok.v[t], t < T: one thread per 8 values
+__global__ void __launch_bounds__(256) k_embed_args(hq_dev_mat W, IdArgs tok, int T, int H, float *__restrict__ x) {
+    const int n = H / 8, i = blockIdx.x * 256 + threadIdx.x, t = i / n, g = i - t * n;
+    if (t >= T) return;
+    float w[8];
+    deq8(W, tok.v[t], g, w);
+    f4 *o = (f4 *)(x + (size_t)t * H + 8 * g);
+    o[0] = f4{w[0], w[1], w[2], w[3]};
+    o[1] = f4{w[4], w[5], w[6], w[7]};
+}
+
 // Readout (src/cuda_backend.cu:561-592, src/cpu_backend.c:253-259): workgroup b normalises the last
-// position x [H] (final RMSNorm, fp32) into LDS and dots it with lm_head row ids[b].
+// position x [H] (final RMSNorm, fp32) into LDS and dots it with lm_head row ids[b] (few.v[b] without ids).
 __global__ void __launch_bounds__(256) k_norm_readout(const float *__restrict__ x, const float *__restrict__ w,
                                                       float off, float eps, hq_dev_mat Wh,
-                                                      const uint32_t *__restrict__ ids, float *__restrict__ logits,
-                                                      int H) {
+                                                      const uint32_t *__restrict__ ids, IdArgs few,
+                                                      float *__restrict__ logits, int H) {
     extern __shared__ float hs[];
     __shared__ float red[4];
     float ss = 0.f;
@@ -222,7 +239,7 @@ __global__ void __launch_bounds__(256) k_norm_readout(const float *__restrict__ 
     const float inv = 1.0f / sqrtf(ss / (float)H + eps);
     for (int i = threadIdx.x; i < H; i += 256) hs[i] = x[i] * inv * (off + w[i]);
     __syncthreads();
-    const size_t r = ids[blockIdx.x];
+    const size_t r = ids ? ids[blockIdx.x] : few.v[blockIdx.x];
     float acc = 0.f;
     for (int g = threadIdx.x; g < H / 8; g += 256) {
         float wv[8];
@@ -240,6 +257,7 @@ unsigned blocks_for(size_t n, unsigned per) { return (unsigned)((n + per - 1) / 
 struct DevLayer {
     hq_mat *q = nullptr, *k = nullptr, *v = nullptr, *o = nullptr, *gate = nullptr, *up = nullptr, *down = nullptr;
     hq_mat *pair = nullptr;  // gate and up as one pair matrix (then gate and up are null)
+    hq_mat *qkv = nullptr;   // q, k and v as one matrix (then q, k and v are null)
     float *in_norm = nullptr, *post_norm = nullptr, *q_norm = nullptr, *k_norm = nullptr;
     float *kc = nullptr, *vc = nullptr;  // [max_seq, kvw] fp32
 };
@@ -256,7 +274,7 @@ struct HipBackend {
     float *x = nullptr, *qb = nullptr, *kb = nullptr, *vb = nullptr, *qr = nullptr, *gb = nullptr, *ub = nullptr;
     _Float16 *hb = nullptr, *ob = nullptr, *fb = nullptr;
     uint32_t *d_tok = nullptr, *d_ids = nullptr;
-    float *d_logits = nullptr, *d_hidden = nullptr;
+    float *h_out = nullptr;  // pinned: logits [MAX_IDS], then the hidden state [H]; kernels write them, no copy
     float *att_part = nullptr;  // partial rows of the attention's split blocks, and their counters
     int *att_cnt = nullptr;
     int n_cu = 0;
@@ -293,10 +311,11 @@ void release(HipBackend *b) {
     (void)hipSetDevice(b->device);
     if (b->st) (void)hipStreamSynchronize(b->st);
     for (DevLayer &l : b->L)
-        for (hq_mat *m : {l.q, l.k, l.v, l.o, l.gate, l.up, l.down, l.pair}) hq_mat_free(m);
+        for (hq_mat *m : {l.q, l.k, l.v, l.o, l.gate, l.up, l.down, l.pair, l.qkv}) hq_mat_free(m);
     if (b->lm_head != b->embed) hq_mat_free(b->lm_head);
     hq_mat_free(b->embed);
     for (void *p : b->allocs) (void)hipFree(p);
+    if (b->h_out) (void)hipHostFree(b->h_out);
     if (b->st) {
         (void)hq_stream_destroy(b->st);  // also frees the stream's GEMM workspace
     }
@@ -344,14 +363,21 @@ int run_layers(HipBackend *b, int T, int pos0) {
         const DevLayer &L = b->L[li];
         k_rmsnorm<_Float16><<<T, 256, 0, st>>>(b->x, L.in_norm, off, eps, b->hb, H);
         BCK(hipGetLastError());
-        if (gemm(b, L.q, b->hb, T, b->qb, false) || gemm(b, L.k, b->hb, T, b->kb, false) ||
-            gemm(b, L.v, b->hb, T, b->vb, false))
+        const float *kb = b->kb, *vb = b->vb;
+        int sq = qw, skv = nkv * hd;
+        if (L.qkv) {
+            if (gemm(b, L.qkv, b->hb, T, b->qb, false)) return -1;
+            kb = b->qb + qw, vb = kb + skv;
+            sq = skv = qw + 2 * skv;
+        } else if (gemm(b, L.q, b->hb, T, b->qb, false) || gemm(b, L.k, b->hb, T, b->kb, false) ||
+                   gemm(b, L.v, b->hb, T, b->vb, false)) {
             return -1;
-        k_qk_rope<<<dim3(T, nh + nkv), 64, 0, st>>>(b->qb, b->kb, b->vb, L.q_norm, L.k_norm, off, eps, b->inv_freq, b->qr,
-                                                    L.kc, L.vc, nh, nkv, hd, (int)c.rot_dim, qw, c.attn_gate, pos0,
+        }
+        k_qk_rope<<<dim3(T, nh + nkv), 64, 0, st>>>(b->qb, kb, vb, L.q_norm, L.k_norm, off, eps, b->inv_freq, b->qr,
+                                                    L.kc, L.vc, nh, nkv, hd, (int)c.rot_dim, sq, skv, skv, c.attn_gate, pos0,
                                                     c.qk_norm);
         BCK(hipGetLastError());
-        const HqAttnArgs at = {b->qr, b->qb, L.kc, L.vc, b->ob, b->att_part, b->att_cnt, T, nh, nkv, hd, qw, c.attn_gate, pos0, scale};
+        const HqAttnArgs at = {b->qr, b->qb, L.kc, L.vc, b->ob, b->att_part, b->att_cnt, T, nh, nkv, hd, sq, c.attn_gate, pos0, scale};
         BCK(hq_launch_attention(at, b->n_cu, st));
         if (gemm(b, L.o, b->ob, T, b->x, true)) return -1;
         k_rmsnorm<_Float16><<<T, 256, 0, st>>>(b->x, L.post_norm, off, eps, b->hb, H);
@@ -388,22 +414,31 @@ int be_forward(hq_ref_backend_t *bb, const uint32_t *tokens, size_t n, const uin
     int last_T = 0;
     for (size_t c0 = 0; c0 < n; c0 += (size_t)b->chunk) {
         const int T = (int)(n - c0 < (size_t)b->chunk ? n - c0 : (size_t)b->chunk);
-        BCK(hipMemcpyAsync(b->d_tok, tokens + c0, (size_t)T * sizeof(uint32_t), hipMemcpyHostToDevice, b->st));
-        BCK(hq_launch_dequant(hq_mat_dev(b->embed), 0, b->d_tok, (uint32_t)T, b->x, b->st));
+        if (T <= 64) {
+            IdArgs tok = {};
+            memcpy(tok.v, tokens + c0, (size_t)T * sizeof(uint32_t));
+            k_embed_args<<<(unsigned)((T * (H / 8) + 255) / 256), 256, 0, b->st>>>(*hq_mat_dev(b->embed), tok, T, H, b->x);
+            BCK(hipGetLastError());
+        } else {
+            BCK(hipMemcpyAsync(b->d_tok, tokens + c0, (size_t)T * sizeof(uint32_t), hipMemcpyHostToDevice, b->st));
+            BCK(hq_launch_dequant(hq_mat_dev(b->embed), 0, b->d_tok, (uint32_t)T, b->x, b->st));
+        }
         if (run_layers(b, T, (int)bb->pos)) return -1;
         bb->pos += (size_t)T;
         last_T = T;
     }
     b->last_T = last_T;
     if (n_ids) {
-        BCK(hipMemcpyAsync(b->d_ids, ids, n_ids * sizeof(uint32_t), hipMemcpyHostToDevice, b->st));
+        IdArgs few = {};
+        if (n_ids <= 64) memcpy(few.v, ids, n_ids * sizeof(uint32_t));
+        else BCK(hipMemcpyAsync(b->d_ids, ids, n_ids * sizeof(uint32_t), hipMemcpyHostToDevice, b->st));
         k_norm_readout<<<n_ids, 256, (size_t)H * sizeof(float), b->st>>>(b->x + (size_t)(last_T - 1) * H, b->final_norm,
                                                                          c.norm_offset, c.eps, *hq_mat_dev(b->lm_head),
-                                                                         b->d_ids, b->d_logits, H);
+                                                                         n_ids <= 64 ? nullptr : b->d_ids, few, b->h_out, H);
         BCK(hipGetLastError());
-        BCK(hipMemcpyAsync(logits, b->d_logits, n_ids * sizeof(float), hipMemcpyDeviceToHost, b->st));
     }
     BCK(hipStreamSynchronize(b->st));
+    if (n_ids) memcpy(logits, b->h_out, n_ids * sizeof(float));
     return 0;
 }
 
@@ -414,10 +449,10 @@ int be_last_hidden(hq_ref_backend_t *bb, float *out) {
     BCK(hipSetDevice(b->device));
     const int H = (int)c.hidden;
     k_rmsnorm<float><<<1, 256, 0, b->st>>>(b->x + (size_t)(b->last_T - 1) * H, b->final_norm, c.norm_offset, c.eps,
-                                           b->d_hidden, H);
+                                           b->h_out + MAX_IDS, H);
     BCK(hipGetLastError());
-    BCK(hipMemcpyAsync(out, b->d_hidden, (size_t)H * sizeof(float), hipMemcpyDeviceToHost, b->st));
     BCK(hipStreamSynchronize(b->st));
+    memcpy(out, b->h_out + MAX_IDS, (size_t)H * sizeof(float));
     return 0;
 }
 
@@ -459,10 +494,26 @@ int init(HipBackend *b, const hq_ref_model_t *m, size_t max_seq) {
         DevLayer &d = b->L[l];
         char what[64];
         snprintf(what, sizeof what, "layer %u", l);
-        if (upload_vec(b, &d.in_norm, s.in_norm, H) || upload_vec(b, &d.post_norm, s.post_norm, H) ||
-            upload_mat(b, &d.q, &s.q, what) || upload_mat(b, &d.k, &s.k, what) || upload_mat(b, &d.v, &s.v, what) ||
-            upload_mat(b, &d.o, &s.o, what) || upload_mat(b, &d.down, &s.down, what))
+        if (upload_vec(b, &d.in_norm, s.in_norm, H) || upload_vec(b, &d.post_norm, s.post_norm, H)) return -1;
+        // q, k and v of one block type and width (and of the config's rows): one matrix. Only types whose GEMM
+        // kernels all hold weights alike: for the others a wider matrix can mean fp16-rounded weights (M > 64)
+        // where three narrow ones had exact ones.
+        const hq_wmat_t *const qkv[3] = {&s.q, &s.k, &s.v};
+        const size_t qrows = (size_t)c.n_heads * hd * (c.attn_gate ? 2 : 1);
+        const int qt = s.q.ggml_type;
+        bool one = (qt == HQ_GGML_Q8_0 || qt == HQ_GGML_Q4_K || qt == HQ_GGML_Q5_K) && s.q.rows == qrows && s.k.rows == kvw && s.v.rows == kvw &&
+                   (qrows + 2 * kvw) * H < ((size_t)1 << 31);
+        for (const hq_wmat_t *w : qkv) one = one && w->dtype == HQ_DT_GGML && w->ggml_type == qt && w->cols == H;
+        if (one) {
+            if (hq_internal_upload_cat(qkv, 3, b->device, &d.qkv)) {
+                char msg[512];
+                snprintf(msg, sizeof msg, "%s", hq_last_error());
+                return hq_internal_fail("hip backend: %s: %s", what, msg);
+            }
+        } else if (upload_mat(b, &d.q, &s.q, what) || upload_mat(b, &d.k, &s.k, what) || upload_mat(b, &d.v, &s.v, what)) {
             return -1;
+        }
+        if (upload_mat(b, &d.o, &s.o, what) || upload_mat(b, &d.down, &s.down, what)) return -1;
         // gate and up of one block type and shape (rows a multiple of 8): one pair matrix
         const bool pair = s.gate.dtype == HQ_DT_GGML && s.up.dtype == HQ_DT_GGML && s.gate.ggml_type == s.up.ggml_type &&
                           s.gate.rows == s.up.rows && s.gate.cols == s.up.cols && s.gate.rows % 8 == 0;
@@ -482,14 +533,14 @@ int init(HipBackend *b, const hq_ref_model_t *m, size_t max_seq) {
     const size_t CH = (size_t)(max_seq < (size_t)CHUNK ? max_seq : (size_t)CHUNK);
     b->chunk = (int)CH;
     const size_t qw = (size_t)c.n_heads * hd * (c.attn_gate ? 2 : 1), ow = (size_t)c.n_heads * hd;
-    if (dalloc(b, (void **)&b->x, CH * H * 4) || dalloc(b, (void **)&b->qb, CH * qw * 4) ||
+    if (dalloc(b, (void **)&b->x, CH * H * 4) || dalloc(b, (void **)&b->qb, CH * (qw + 2 * kvw) * 4) ||
         dalloc(b, (void **)&b->kb, CH * kvw * 4) || dalloc(b, (void **)&b->vb, CH * kvw * 4) ||
         dalloc(b, (void **)&b->qr, CH * ow * 4) || dalloc(b, (void **)&b->gb, CH * I * 4) ||
         dalloc(b, (void **)&b->ub, CH * I * 4) || dalloc(b, (void **)&b->hb, CH * H * 2) ||
         dalloc(b, (void **)&b->ob, CH * ow * 2) || dalloc(b, (void **)&b->fb, CH * I * 2) ||
-        dalloc(b, (void **)&b->d_tok, CH * 4) || dalloc(b, (void **)&b->d_ids, MAX_IDS * 4) ||
-        dalloc(b, (void **)&b->d_logits, MAX_IDS * 4) || dalloc(b, (void **)&b->d_hidden, H * 4))
+        dalloc(b, (void **)&b->d_tok, CH * 4) || dalloc(b, (void **)&b->d_ids, MAX_IDS * 4))
         return -1;
+    BCK(hipHostMalloc((void **)&b->h_out, (MAX_IDS + H) * sizeof(float), hipHostMallocDefault));
     BCK(hipDeviceGetAttribute(&b->n_cu, hipDeviceAttributeMultiprocessorCount, b->device));
     if (dalloc(b, (void **)&b->att_part, hq_attn_work_bytes((int)hd, b->n_cu)) ||
         dalloc(b, (void **)&b->att_cnt, HQ_ATTN_MAX_BLOCKS * sizeof(int)))
@@ -503,12 +554,12 @@ int init(HipBackend *b, const hq_ref_model_t *m, size_t max_seq) {
             const hq_mat *w;
             uint32_t rows, cols;
             const char *name;
-        } want[] = {{d.q, (uint32_t)qw, (uint32_t)H, "q"},        {d.k, (uint32_t)kvw, (uint32_t)H, "k"},
+        } want[] = {{d.qkv, (uint32_t)(qw + 2 * kvw), (uint32_t)H, "q/k/v"}, {d.q, (uint32_t)qw, (uint32_t)H, "q"},        {d.k, (uint32_t)kvw, (uint32_t)H, "k"},
                     {d.v, (uint32_t)kvw, (uint32_t)H, "v"},        {d.o, (uint32_t)H, (uint32_t)ow, "o"},
                     {d.gate, (uint32_t)I, (uint32_t)H, "gate"},   {d.up, (uint32_t)I, (uint32_t)H, "up"},
                     {d.pair, 2 * (uint32_t)I, (uint32_t)H, "gate/up"}, {d.down, (uint32_t)H, (uint32_t)I, "down"}};
         for (auto &w : want) {
-            if (!w.w) continue;  // (gate and up, or their pair)
+            if (!w.w) continue;  // (q, k and v, gate and up, or what holds them together)
             if (hq_mat_shape(w.w, &r, &k, nullptr)) return -1;
             if (r != w.rows || k != w.cols)
                 return hq_internal_fail("hip backend: layer %u %s is [%u, %u], the config needs [%u, %u]", l, w.name, r, k,
@@ -753,7 +804,7 @@ extern "C" int hip_selftest(const hq_ref_model_t *m, int device, size_t n_tokens
     int failed = 0, rc = 0;
     printf("hq_gemm on the model's matrices vs a float64 host product of the decoded weights:\n");
     const DevLayer &L0 = b->L[0];
-    rc = selftest_gemm(L0.q, "q", verbose, &failed, b->st) || selftest_gemm(L0.down, "down", verbose, &failed, b->st) ||
+    rc = selftest_gemm(L0.qkv ? L0.qkv : L0.q, L0.qkv ? "qkv" : "q", verbose, &failed, b->st) || selftest_gemm(L0.down, "down", verbose, &failed, b->st) ||
          (!L0.pair && selftest_gemm(L0.gate, "gate", verbose, &failed, b->st));
     if (L0.pair) {
         printf("hq_gemm_swiglu on the gate/up pair vs silu(g) * u from the decoded weights in float64:\n");

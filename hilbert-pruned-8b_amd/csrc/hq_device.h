@@ -223,6 +223,11 @@ DEV h2 bytes_f16(uint32_t w, bool hi_pair) {
 // pair matrix, fp16 (see tile_finish).
 constexpr int HQ_OUT_SWIGLU = 2;
 
+// fp16(silu(g) * u), as the separate pass over a product computes it; output i of a pair matrix comes from
+// its rows pair_row(i) (gate) and pair_row(i) + 8 (up)
+DEV uint16_t swiglu_f16(float g, float u) { return __builtin_bit_cast(uint16_t, (_Float16)(g / (1.0f + expf(-g)) * u)); }
+DEV int pair_row(int i) { return 16 * (i >> 3) + (i & 7); }
+
 // SwiGLU output from accumulators in the MFMA layout of the register-decode kernels (lane (ln, lg) of
 // block (i, j): row 16i + ln, columns 16j + 4lg .. + 3 of the wave's columns). Each 16-column block of
 // a gate/up pair matrix is 8 gate columns and the 8 matching up columns, so lanes 32 apart hold

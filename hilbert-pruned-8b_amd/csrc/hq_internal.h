@@ -4,6 +4,8 @@
 
 #include <stdint.h>
 
+#include "hq.h"
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -15,6 +17,9 @@ int hq_internal_fail(const char *fmt, ...) __attribute__((format(printf, 1, 2)))
 int hq_internal_block_shape(int ggml_type, uint32_t *values, uint32_t *bytes);
 /* The accepted block types, for messages ("Q8_0 = 8, ..."). */
 const char *hq_internal_supported_types(void);
+
+/* The rows of n matrices of one type and width (Hugging Face order, one after the other) as one resident matrix. */
+int hq_internal_upload_cat(const hq_wmat_t *const *w, int n, int device, hq_mat **out);
 
 #ifdef __cplusplus
 }

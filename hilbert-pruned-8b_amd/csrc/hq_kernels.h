@@ -35,6 +35,9 @@ int hq_mat_device(const struct hq_mat *m);
 hipError_t hq_launch_dequant(const hq_dev_mat *W, uint32_t row0, const uint32_t *ids, uint32_t nrows, float *out,
                              hipStream_t st);
 hipError_t hq_launch_gemv(const hq_dev_mat *W, const uint16_t *a, void *C, int c_f32, int accumulate, hipStream_t st);
+// M = 1 of a gate/up pair matrix: out[i] = fp16(silu(gate_i . a) * (up_i . a)), the GEMV kernels' dots and
+// the product in their epilogue (*fused = 0: no such kernel for the shape, nothing was launched)
+hipError_t hq_launch_gemv_pair(const hq_dev_mat *W, const uint16_t *a, uint16_t *out, hipStream_t st, int *fused);
 // Stream-K workspace: fp32 partial tiles and per-tile counters (zero when idle; each launch leaves
 // them zero), the activation sub-block sums of the wide Q4_K kernel, and the number of CUs the
 // persistent grid is sized for.
@@ -139,6 +142,7 @@ hipError_t hq_launch_dequant_q6k(const hq_dev_mat *W, uint32_t row0, const uint3
 hipError_t hq_launch_dequant_kq(const hq_dev_mat *W, uint32_t row0, const uint32_t *ids, uint32_t nrows, float *out,
                                 hipStream_t st);
 hipError_t hq_launch_gemv_kq(const hq_dev_mat *W, const uint16_t *a, void *C, int c_f32, int accumulate, hipStream_t st);
+hipError_t hq_launch_gemv_pair_kq(const hq_dev_mat *W, const uint16_t *a, uint16_t *out, hipStream_t st);
 int hq_sb_rows(int n_out);       // rows per wave of that GEMV and gather for n_out rows
 int hq_sb_lds(int type, int K);  // whether that GEMV copies its activation vector into LDS
 hipError_t hq_launch_gather_kq(const hq_dev_mat *W, const uint16_t *H, const uint32_t *ids, int B, int k, float *out,

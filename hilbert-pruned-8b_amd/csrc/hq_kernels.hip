@@ -339,7 +339,13 @@ __global__ void __launch_bounds__(256) k_gemv_q4_k_s(const uint8_t *__restrict__
     if (lane < R) red[wave * R + lane] = acc;
     __syncthreads();
     const int n = blockIdx.x * R + tid;
-    if (tid < R && n < N) store_out(C, n, ((red[tid] + red[R + tid]) + red[2 * R + tid]) + red[3 * R + tid], c_f32, accumulate);
+    const float v = tid < R ? ((red[tid] + red[R + tid]) + red[2 * R + tid]) + red[3 * R + tid] : 0.f;
+    if (R >= 16 && c_f32 == HQ_OUT_SWIGLU) {  // pair matrix: rows 16 k + e (gate) and 16 k + 8 + e (up) of the slab
+        const float u = __shfl(v, tid + 8, 64);
+        if (tid < R && !(tid & 8) && n < N) ((uint16_t *)C)[(n >> 4) * 8 + (n & 7)] = swiglu_f16(v, u);
+        return;
+    }
+    if (tid < R && n < N) store_out(C, n, v, c_f32, accumulate);
 }
 
 // ---- Q4_K GEMV (M = 1), streamed: a workgroup owns 8 weight rows; its S waves split the row's
@@ -350,7 +356,8 @@ __global__ void __launch_bounds__(256) k_gemv_q4_k_s(const uint8_t *__restrict__
 // lane (row = lane / 8, j = lane % 8) takes the unit j = 32-byte quant group j % 4 of super-block
 // j / 4 (64 values: low nibbles sub-block 2p, high nibbles 2p + 1), dotted by gemv_unit_q4_k.
 // The activations and their 32-value sub-block sums are staged once per workgroup. Row totals:
-// 8-lane butterfly, then the S wave partials in wave order. Needs an even number of super-blocks
+// 8-lane butterfly, then the S wave partials in wave order. SwiGLU of a pair matrix: 2 S waves, the second
+// half on the next 8 rows (the up rows of the first half's gate rows). Needs an even number of super-blocks
 // per row.
 constexpr int GVR_SLOT = 8 * 288;
 
@@ -359,18 +366,20 @@ __global__ void __launch_bounds__(256) k_gemv_q4_k_r(const uint8_t *__restrict__
                                                      const uint16_t *__restrict__ a, int N, int K, void *C, int c_f32,
                                                      int accumulate) {
     extern __shared__ __attribute__((aligned(16))) char gr_lds[];
-    const int tid = threadIdx.x, lane = tid & 63, S = (int)blockDim.x >> 6;
+    const bool pair = c_f32 == HQ_OUT_SWIGLU;
+    const int tid = threadIdx.x, lane = tid & 63, NW = (int)blockDim.x >> 6, S = pair ? NW / 2 : NW;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar control flow
+    const int grp = wave >= S ? 1 : 0, ws = wave - grp * S;
     const uint32_t act_bytes = 2u * (uint32_t)K;
     char *const sa = gr_lds;
     float *const ss = (float *)(gr_lds + act_bytes);  // K / 32 sub-block sums
-    float *const red = ss + K / 32;                   // [S][8] wave partials
-    char *const ring = (char *)(red + 8 * S) + (size_t)wave * NS * GVR_SLOT;
+    float *const red = ss + K / 32;                   // [NW][8] wave partials
+    char *const ring = (char *)(red + 8 * NW) + (size_t)wave * NS * GVR_SLOT;
     const uint32_t lds0 = (uint32_t)(uintptr_t)gr_lds;
     const rsrc_t ra = make_rsrc(a, act_bytes);
     const rsrc_t rw = make_rsrc(W, (uint32_t)N * row_bytes);  // rows >= N read as zero
-    const int n0 = blockIdx.x * 8, pairs = K / 512;
-    const int pr0 = wave * pairs / S, nst = (wave + 1) * pairs / S - pr0;
+    const int n0 = (pair ? 2 * blockIdx.x + grp : blockIdx.x) * 8, pairs = K / 512;
+    const int pr0 = ws * pairs / S, nst = (ws + 1) * pairs / S - pr0;
     // this lane's gather offsets for the three DMA instructions of a stage (lane l = 64 q + lane of
     // the stage: row l / 18, 16-byte piece l % 18)
     uint32_t dvo[3];
@@ -388,13 +397,13 @@ __global__ void __launch_bounds__(256) k_gemv_q4_k_r(const uint8_t *__restrict__
     };
     // activations (this wave's share of the 1 KB pieces), then the first NS stages
     int nact = 0;
-    for (uint32_t o = 1024u * wave; o < act_bytes; o += 1024u * S, nact++)
+    for (uint32_t o = 1024u * wave; o < act_bytes; o += 1024u * NW, nact++)
         if (o + 16u * lane < act_bytes) dma16_untracked(ra, lds0 + o, o + 16u * lane);
     const int pre = nst < NS ? nst : NS;
     for (int st = 0; st < pre; st++) issue(st);
     wait_vmcnt(3 * pre);
     __syncthreads();
-    for (int i = tid; i < K / 32; i += 64 * S) {
+    for (int i = tid; i < K / 32; i += 64 * NW) {
         const u4v *p = (const u4v *)(sa + 64 * i);
         ss[i] = sum8(p[3], sum8(p[2], sum8(p[1], sum8(p[0], 0.f))));
     }
@@ -414,7 +423,7 @@ __global__ void __launch_bounds__(256) k_gemv_q4_k_r(const uint8_t *__restrict__
     acc += __shfl_xor(acc, 1, 64);
     acc += __shfl_xor(acc, 2, 64);
     acc += __shfl_xor(acc, 4, 64);
-    if (S == 1) {
+    if (NW == 1) {
         if (j == 0 && n0 + row < N) store_out(C, n0 + row, acc, c_f32, accumulate);
         return;
     }
@@ -423,7 +432,13 @@ __global__ void __launch_bounds__(256) k_gemv_q4_k_r(const uint8_t *__restrict__
     if (tid < 8 && n0 + tid < N) {
         float v = red[tid];
         for (int w = 1; w < S; w++) v += red[w * 8 + tid];
-        store_out(C, n0 + tid, v, c_f32, accumulate);
+        if (pair) {
+            float u = red[8 * S + tid];
+            for (int w = 1; w < S; w++) u += red[(S + w) * 8 + tid];
+            ((uint16_t *)C)[8 * blockIdx.x + tid] = swiglu_f16(v, u);
+        } else {
+            store_out(C, n0 + tid, v, c_f32, accumulate);
+        }
     }
 }
 
@@ -443,6 +458,18 @@ __global__ void __launch_bounds__(256) k_gemv_q8_0(const uint8_t *__restrict__ q
         const float v = row_sum<64>(acc[r]);
         if (j == 0 && n0 + r < N) store_out(C, n0 + r, v, c_f32, accumulate);
     }
+}
+
+// SwiGLU of a pair matrix, M = 1: a wave per output, its gate and up rows together
+__global__ void __launch_bounds__(256) k_gemv_q8_0_pair(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ d, int ldd,
+                                                        const uint16_t *__restrict__ a, int I, int K, uint16_t *__restrict__ out) {
+    const int j = threadIdx.x & 63, i = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (i >= I) return;
+    const int n[2] = {pair_row(i), pair_row(i) + 8};
+    float acc[2];
+    rows_q8_0<2>(qs, d, ldd, a, K, n, j, acc);
+    const float g = row_sum<64>(acc[0]), u = row_sum<64>(acc[1]);
+    if (j == 0) out[i] = swiglu_f16(g, u);
 }
 
 template <int R>
@@ -873,6 +900,34 @@ hipError_t hq_launch_gemv(const hq_dev_mat *W, const uint16_t *a, void *C, int c
         launch_gemv_t<1>(W, a, C, c_f32, accumulate, st);
     }
     return hipGetLastError();
+}
+
+hipError_t hq_launch_gemv_pair(const hq_dev_mat *W, const uint16_t *a, uint16_t *out, hipStream_t st, int *fused) {
+    const int N = (int)W->rows, K = (int)W->cols, I = N / 2;
+    const size_t rb = W->row_bytes;
+    *fused = 1;
+    if (W->type == HQ_TYPE_Q6_K || hq_is_kq(W->type)) return hq_launch_gemv_pair_kq(W, a, out, st);
+    if (W->type == HQ_TYPE_Q8_0) {
+        k_gemv_q8_0_pair<<<(I + 3) / 4, 256, 0, st>>>(W->qs, W->d, W->ldd, a, I, K, out);
+        return hipGetLastError();
+    }
+    const GemvPlan pl = gemv_plan(W);
+    const size_t fixed = (size_t)K * 2 + K / 32 * 4;
+    if (pl.kind == GemvPlan::Q4K_STREAM) {  // two row groups per workgroup
+        const size_t lds = fixed + 2 * (pl.lds - fixed);
+        if (lds <= 64 * 1024) {
+            k_gemv_q4_k_r<GVR_NS><<<N / 16, 2 * 64 * pl.r, lds, st>>>(W->qs, (uint32_t)rb, a, N, K, out, HQ_OUT_SWIGLU, 0);
+            return hipGetLastError();
+        }
+    }
+    // a slab of 16 rows: 8 gate rows and their up rows
+    const size_t lds = fixed + 16 * (rb + 16);
+    if (lds <= 64 * 1024 && ((size_t)N + 32) * rb < ((size_t)1 << 32)) {
+        k_gemv_q4_k_s<16><<<N / 16, 256, lds, st>>>(W->qs, (uint32_t)rb, a, N, K, out, HQ_OUT_SWIGLU, 0);
+        return hipGetLastError();
+    }
+    *fused = 0;
+    return hipSuccess;
 }
 
 template <int LPR>
@@ -1422,8 +1477,7 @@ hipError_t hq_launch_gemm_swiglu(const hq_dev_mat *W, const uint16_t *A, int M, 
 __global__ void __launch_bounds__(256) k_swiglu_pairs(const float *__restrict__ C, uint16_t *__restrict__ out, size_t n_out) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n_out; i += (size_t)gridDim.x * blockDim.x) {
         const size_t k = i / 8, e = i % 8;
-        const float g = C[16 * k + e], u = C[16 * k + 8 + e];
-        out[i] = __builtin_bit_cast(uint16_t, (_Float16)(g / (1.0f + expf(-g)) * u));
+        out[i] = swiglu_f16(C[16 * k + e], C[16 * k + 8 + e]);
     }
 }
 

@@ -188,9 +188,12 @@ __global__ void __launch_bounds__(256) k_gemv_sb(const uint8_t *__restrict__ W, 
     extern __shared__ __attribute__((aligned(16))) uint16_t sb_act[];
     constexpr int S = 8 / RW, G = 8 * S;  // super-blocks side by side, lanes per row
     const int lane = threadIdx.x & 63, o0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RW;
-    if (!LDSA && o0 >= n_out) return;
-    const int p = lane & 7, s = (lane >> 3) & (S - 1), o = o0 + lane / G, oc = min(o, n_out - 1);
-    uint32_t row = (uint32_t)oc;
+    if (!LDSA && o0 >= (RW == 2 && !GATHER && c_f32 == HQ_OUT_SWIGLU ? 2 * n_out : n_out)) return;
+    // SwiGLU of a pair matrix (RW = 2, N = 2 n_out rows): a wave per output, its gate row in the lower lanes and
+    // its up row in the upper ones
+    const bool pair = RW == 2 && !GATHER && c_f32 == HQ_OUT_SWIGLU;
+    const int p = lane & 7, s = (lane >> 3) & (S - 1), o = pair ? o0 / 2 : o0 + lane / G, oc = min(o, n_out - 1);
+    uint32_t row = pair ? (uint32_t)(pair_row(oc) + 8 * (lane / G)) : (uint32_t)oc;
     const uint16_t *av = a;
     if constexpr (GATHER) {
         const uint32_t id = ids[oc];
@@ -209,7 +212,7 @@ __global__ void __launch_bounds__(256) k_gemv_sb(const uint8_t *__restrict__ W, 
     }();
     if constexpr (LDSA) {
         __syncthreads();
-        if (o0 >= n_out) return;  // (waves past n_out leave after the barrier)
+        if (pair ? o >= n_out : o0 >= n_out) return;  // (waves past n_out leave after the barrier)
     }
     sb_load_a<T>(x, act + 256 * u, p);
     for (u = s; u < nsb; u += S) {
@@ -222,6 +225,11 @@ __global__ void __launch_bounds__(256) k_gemv_sb(const uint8_t *__restrict__ W, 
     }
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (pair) {
+        const float u = __shfl(acc, G, 64);
+        if (lane == 0 && o < n_out) ((uint16_t *)C)[o] = swiglu_f16(acc, u);
+        return;
+    }
     if ((lane & (G - 1)) == 0 && o < n_out) {
         if constexpr (GATHER) ((float *)C)[o] = ids[o] < rows ? acc : __builtin_nanf("");
         else store_out(C, (size_t)o, acc, c_f32, accumulate);
@@ -293,6 +301,24 @@ hipError_t hq_launch_gemv_kq(const hq_dev_mat *W, const uint16_t *a, void *C, in
     case HQ_TYPE_Q6_K: return launch_sb<HQ_TYPE_Q6_K, false>(W, a, nullptr, n, 1, C, c_f32, accumulate, st);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t hq_launch_gemv_pair_kq(const hq_dev_mat *W, const uint16_t *a, uint16_t *out, hipStream_t st) {
+    const int I = (int)W->rows / 2, K = (int)W->cols;
+    const unsigned grid = (unsigned)((I + 3) / 4);
+#define PAIR(t)                                                                                                           \
+    if (hq_sb_lds(t, K)) k_gemv_sb<t, 2, false, true><<<grid, 256, (size_t)K * 2, st>>>(W->qs, W->row_bytes, a, nullptr, I, 1, K, W->rows, \
+                                                                                       out, HQ_OUT_SWIGLU, 0);             \
+    else k_gemv_sb<t, 2, false, false><<<grid, 256, 0, st>>>(W->qs, W->row_bytes, a, nullptr, I, 1, K, W->rows, out, HQ_OUT_SWIGLU, 0)
+    switch (W->type) {
+    case HQ_TYPE_Q2_K: PAIR(HQ_TYPE_Q2_K); break;
+    case HQ_TYPE_Q3_K: PAIR(HQ_TYPE_Q3_K); break;
+    case HQ_TYPE_Q5_K: PAIR(HQ_TYPE_Q5_K); break;
+    case HQ_TYPE_Q6_K: PAIR(HQ_TYPE_Q6_K); break;
+    default: return hipErrorInvalidValue;
+    }
+#undef PAIR
+    return hipGetLastError();
 }
 
 hipError_t hq_launch_gather_kq(const hq_dev_mat *W, const uint16_t *H, const uint32_t *ids, int B, int k, float *out,

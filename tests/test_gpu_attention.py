@@ -39,3 +39,19 @@ def test_attention_edges(hqlib, oracle, nh, nkv, hd, prefix, T):
     print(f"[gpu] attention {nh}/{nkv} x {hd}, {prefix} + {T}: max_abs {max_abs(got, ref):.2e}", flush=True)
     assert max_abs(got, ref) <= 1e-2
     assert again is None or max_abs(again, got) <= 1e-3
+
+
+def test_many_ids_and_long_prompts(hqlib, oracle):
+    """Token and id counts on both sides of what a launch carries as arguments (64): the same logits for the
+    same ids, the oracle's within the bar."""
+    cfg = dict(synth.TINY_LLAMA, n_layers=1, hidden=256, intermediate=256, vocab=512, n_heads=4, n_kv_heads=2, head_dim=64)
+    model = synth.tiny_llama(9, cfg)
+    tokens, ids = synth.tiny_llama_prompt(8, T=129, vocab=512, n_ids=65)
+    be = hqlib.HipBackend(hqlib.RefModelView(model), 129)
+    many = be.forward(tokens, ids)
+    be.reset()
+    be.forward(tokens[:65])
+    few = be.forward(tokens[65:], ids[:64])
+    be.destroy()
+    ref = oracle.llama_forward(model, tokens, ids)
+    assert max_abs(many, ref) <= 1e-2 and max_abs(few, many[:64]) <= 1e-3

@@ -51,7 +51,7 @@ def test_small_tiles(hqlib, oracle, gtype, M, N, K):
 
 
 @pytest.mark.parametrize("gtype", TYPES)
-@pytest.mark.parametrize("M,I,K", [(2, 24, 512), (16, 200, 256), (33, 1000, 768), (64, 72, 2560)])
+@pytest.mark.parametrize("M,I,K", [(1, 24, 512), (1, 200, 256), (1, 4104, 1024), (2, 24, 512), (16, 200, 256), (33, 1000, 768), (64, 72, 2560)])
 def test_small_tiles_swiglu(hqlib, oracle, gtype, M, I, K):
     g, u = (synth.random_blocks(gtype, synth.Rng(41 + I + i), I, K) for i in (0, 1))
     a = synth.activations_f16(synth.Rng(42 + M), M, K)
