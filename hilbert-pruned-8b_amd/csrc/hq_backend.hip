@@ -30,6 +30,7 @@
 #include <stdlib.h>
 #include <string.h>
 #include <time.h>
+#include <algorithm>
 #include <vector>
 
 #include "hq.h"
@@ -49,7 +50,9 @@ namespace {
             return hq_internal_fail("HIP %s failed: %s (%s:%d)", #call, hipGetErrorString(e_), __FILE__, __LINE__); \
     } while (0)
 
-constexpr int CHUNK = 1024;    // tokens per layer-loop pass
+// tokens per layer-loop pass: of 2048 the row blocks of attention share the CUs (512 of 32 rows, longest first)
+// and each weight is decoded once. 4 layers of 512, 2048 tokens: 803 us in two passes of 1024, 590 in one.
+constexpr int CHUNK = 2048;
 constexpr int MAX_IDS = 4096;  // readout ids per forward
 
 // Up to 64 tokens or readout ids as a kernel argument: a copy of them to the device costs a launch of its own.
@@ -130,58 +133,67 @@ __global__ void __launch_bounds__(256) k_rmsnorm(const float *__restrict__ x, co
     for (int i = threadIdx.x; i < H; i += 256) out[(size_t)blockIdx.x * H + i] = (T)(xr[i] * inv * (off + w[i]));
 }
 
-// One wave per (token t, head j): heads j < nh are queries (q rows of qb, [q | gate]
-// per head when gated), the others keys of kv head j - nh (whose value row is copied alongside).
-// Optional q/k RMSNorm, then RoPE on the first rot dims (pairs i, i + rot/2) at position pos0 + t
-// (src/cpu_backend.c:86-102). Queries go to qr [T, nh, hd]; keys and values to the caches.
-// sq, sk, sv: row strides of qb, kb, vb.
-__global__ void __launch_bounds__(64) k_qk_rope(const float *__restrict__ qb, const float *__restrict__ kb,
+// A workgroup of ROPE_W waves takes token t and heads ROPE_W y + w, ROPE_W (y + gridDim.y) + w, ..., a wave
+// at a time: heads j < nh are queries (q rows of qb, [q | gate] per head when gated), the others keys of
+// kv head j - nh (whose value row is copied alongside). Optional q/k RMSNorm, then RoPE on the first rot
+// dims (pairs i, i + rot/2) at position pos0 + t (src/cpu_backend.c:86-102). Queries go to qr [T, nh, hd];
+// keys and values to the caches. sq, sk, sv: row strides of qb, kb, vb.
+// Bound: the angles' sines and cosines, formed once per workgroup for all of its heads, and for one token
+// the chain of reads. 2048 tokens, 8 + 8 heads of 64: 12.0 us with a workgroup and its own angles per head -> 8.6 us.
+constexpr int ROPE_W = 4;
+__global__ void __launch_bounds__(64 * ROPE_W) k_qk_rope(const float *__restrict__ qb, const float *__restrict__ kb,
                                                 const float *__restrict__ vb, const float *__restrict__ qn,
                                                 const float *__restrict__ kn, float off, float eps,
                                                 const float *__restrict__ inv_freq, float *__restrict__ qr,
                                                 float *__restrict__ kc, float *__restrict__ vc, int nh, int nkv, int hd,
                                                 int rot, int sq, int sk, int sv, int gated, int pos0, int qk_norm) {
-    __shared__ float xs[256];
-    const int t = blockIdx.x, j = blockIdx.y, lane = threadIdx.x, kvw = nkv * hd;
-    const bool is_q = j < nh;
-    const float *src = is_q ? qb + (size_t)t * sq + (size_t)j * hd * (gated ? 2 : 1) : kb + (size_t)t * sk + (size_t)(j - nh) * hd;
-    float *dst = is_q ? qr + ((size_t)t * nh + j) * hd : kc + (size_t)(pos0 + t) * kvw + (size_t)(j - nh) * hd;
-    float v[4];
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int d = lane + 64 * i;
-        v[i] = d < hd ? src[d] : 0.f;
-        ss += v[i] * v[i];
+    __shared__ float cs[128], sn[128], xs[ROPE_W][256];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, kvw = nkv * hd, half = rot / 2;
+    const float p = (float)(pos0 + t);
+    for (int f = threadIdx.x; f < half; f += 64 * ROPE_W) {
+        const float a = inv_freq[f] * p;
+        cs[f] = cosf(a), sn[f] = sinf(a);
     }
-    if (qk_norm) {
-        ss = wave_sum(ss);
-        const float inv = 1.0f / sqrtf(ss / (float)hd + eps);
-        const float *nw = is_q ? qn : kn;
+    for (int j0 = ROPE_W * blockIdx.y; j0 < nh + nkv; j0 += ROPE_W * gridDim.y) {
+        const int j = j0 + w;
+        const bool on = j < nh + nkv, is_q = j < nh;
+        const float *src = is_q ? qb + (size_t)t * sq + (size_t)j * hd * (gated ? 2 : 1) : kb + (size_t)t * sk + (size_t)(j - nh) * hd;
+        float *dst = is_q ? qr + ((size_t)t * nh + j) * hd : kc + (size_t)(pos0 + t) * kvw + (size_t)(j - nh) * hd;
+        float v[4];
+        float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int d = lane + 64 * i;
-            if (d < hd) v[i] = v[i] * inv * (off + nw[d]);
+            v[i] = on && d < hd ? src[d] : 0.f;
+            ss += v[i] * v[i];
         }
-    }
+        if (qk_norm) {
+            ss = wave_sum(ss);
+            const float inv = 1.0f / sqrtf(ss / (float)hd + eps);
+            const float *nw = is_q ? qn : kn;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (lane + 64 * i < hd) xs[lane + 64 * i] = v[i];
-    __syncthreads();
-    const float p = (float)(pos0 + t);
-    const int half = rot / 2;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int d = lane + 64 * i;
-        if (d >= hd) continue;
-        float y = xs[d];
-        if (d < rot) {
-            const int f = d < half ? d : d - half;
-            const float a = inv_freq[f] * p, cs = cosf(a), sn = sinf(a);
-            y = d < half ? xs[d] * cs - xs[d + half] * sn : xs[d] * cs + xs[d - half] * sn;
+            for (int i = 0; i < 4; i++) {
+                const int d = lane + 64 * i;
+                if (d < hd) v[i] = v[i] * inv * (off + nw[d]);
+            }
         }
-        dst[d] = y;
-        if (!is_q) vc[(size_t)(pos0 + t) * kvw + (size_t)(j - nh) * hd + d] = vb[(size_t)t * sv + (size_t)(j - nh) * hd + d];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (lane + 64 * i < hd) xs[w][lane + 64 * i] = v[i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int d = lane + 64 * i;
+            if (!on || d >= hd) continue;
+            float y = v[i];
+            if (d < rot) {
+                const int f = d < half ? d : d - half;
+                y = d < half ? v[i] * cs[f] - xs[w][d + half] * sn[f] : v[i] * cs[f] + xs[w][d - half] * sn[f];
+            }
+            dst[d] = y;
+            if (!is_q) vc[(size_t)(pos0 + t) * kvw + (size_t)(j - nh) * hd + d] = vb[(size_t)t * sv + (size_t)(j - nh) * hd + d];
+        }
+        __syncthreads();
     }
 }
 
@@ -373,9 +385,11 @@ int run_layers(HipBackend *b, int T, int pos0) {
                    gemm(b, L.v, b->hb, T, b->vb, false)) {
             return -1;
         }
-        k_qk_rope<<<dim3(T, nh + nkv), 64, 0, st>>>(b->qb, kb, vb, L.q_norm, L.k_norm, off, eps, b->inv_freq, b->qr,
-                                                    L.kc, L.vc, nh, nkv, hd, (int)c.rot_dim, sq, skv, skv, c.attn_gate, pos0,
-                                                    c.qk_norm);
+        // few tokens: their heads over several workgroups, while there are fewer than 8 per CU
+        const int rope_y = std::min((nh + nkv + ROPE_W - 1) / ROPE_W, std::max(8 * b->n_cu / T, 1));
+        k_qk_rope<<<dim3(T, rope_y), 64 * ROPE_W, 0, st>>>(b->qb, kb, vb, L.q_norm, L.k_norm, off, eps, b->inv_freq, b->qr,
+                                                           L.kc, L.vc, nh, nkv, hd, (int)c.rot_dim, sq, skv, skv,
+                                                           c.attn_gate, pos0, c.qk_norm);
         BCK(hipGetLastError());
         const HqAttnArgs at = {b->qr, b->qb, L.kc, L.vc, b->ob, b->att_part, b->att_cnt, T, nh, nkv, hd, sq, c.attn_gate, pos0, scale};
         BCK(hq_launch_attention(at, b->n_cu, st));

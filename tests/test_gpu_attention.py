@@ -55,3 +55,21 @@ def test_many_ids_and_long_prompts(hqlib, oracle):
     be.destroy()
     ref = oracle.llama_forward(model, tokens, ids)
     assert max_abs(many, ref) <= 1e-2 and max_abs(few, many[:64]) <= 1e-3
+
+
+@pytest.mark.parametrize("nh,nkv,rot,T", [(3, 1, 64, 2049), (5, 1, 32, 2150), (2, 2, 64, 1537), (3, 3, 16, 3)])
+def test_passes_of_a_long_prompt(hqlib, oracle, nh, nkv, rot, T):
+    """Prompts around one pass of the layer loop (2048 tokens; 2049 leaves a pass of one token), head counts
+    that do not fill the rotary kernel's workgroups, and fewer rotated dims than the head has."""
+    cfg = dict(synth.TINY_LLAMA, n_layers=1, hidden=256, intermediate=256, vocab=512, n_heads=nh, n_kv_heads=nkv, head_dim=64,
+               rot_dim=rot)
+    model = synth.tiny_llama(nh + T, cfg)
+    tokens, ids = synth.tiny_llama_prompt(11, T=T, vocab=512, n_ids=16)
+    be = hqlib.HipBackend(hqlib.RefModelView(model), T)
+    got = be.forward(tokens, ids)
+    be.reset()
+    be.forward(tokens[: T // 2])
+    split = be.forward(tokens[T // 2:], ids)
+    be.destroy()
+    ref = oracle.llama_forward(model, tokens, ids)
+    assert max_abs(got, ref) <= 1e-2 and max_abs(split, got) <= 1e-3
