@@ -676,7 +676,7 @@ namespace {
 // The K split's sum: the parts' tiles (tile_finish's layout: 16-byte piece h of 8-value chunk c of
 // tile t, part p at ((t parts + p) TILE) + (h NCH + c) 16 bytes) added in part order, as tile_finish's
 // last part would, by one thread per chunk over all CUs, then stored to C
-template <int BN>
+template <int BN, int MAXP>
 __global__ void __launch_bounds__(256) k_tile_reduce(const float *__restrict__ partials, int parts, int ntiles, int mt,
                                                      int M, int N, void *C, int c_f32, int accumulate) {
     constexpr int CH = BN / 8, NCH = WR_BM * CH;
@@ -687,13 +687,16 @@ __global__ void __launch_bounds__(256) k_tile_reduce(const float *__restrict__ p
     const int nt_i = tile / mt, mt_i = tile - nt_i * mt, m = mt_i * WR_BM + row, n = nt_i * BN + 8 * ch;
     if (m >= M || n >= N) return;
     const char *base = (const char *)partials + (size_t)tile * parts * TILE + (size_t)c * 16;
-    f4 pv[4][2];
+    f4 pv[MAXP][2];
 #pragma unroll
-    for (int p = 0; p < 4; p++)
-        if (p < parts) pv[p][0] = *(const f4 *)(base + p * TILE), pv[p][1] = *(const f4 *)(base + p * TILE + NCH * 16);
+    for (int p = 0; p < MAXP; p++)
+        if (MAXP > 4 || p < parts) {  // (with more than 4, most are there: the rest read the last again)
+            const char *q = base + (size_t)(MAXP > 4 ? min(p, parts - 1) : p) * TILE;
+            pv[p][0] = *(const f4 *)q, pv[p][1] = *(const f4 *)(q + NCH * 16);
+        }
     f4 v0 = f4{0.f, 0.f, 0.f, 0.f}, v1 = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int p = 0; p < 4; p++)
+    for (int p = 0; p < MAXP; p++)
         if (p < parts) v0 += pv[p][0], v1 += pv[p][1];
     const bool wide = (N & 7) == 0 && ((uintptr_t)C & 15u) == 0;
     store8_out(C, N, m, n, v0, v1, wide, c_f32, accumulate);
@@ -705,10 +708,11 @@ __global__ void __launch_bounds__(256) k_tile_reduce(const float *__restrict__ p
 // separate sum measured slower there, e.g. Q8_0 M = 128, N = 9728, two parts: 19.2 -> 20.3 us.)
 hipError_t hq_launch_tile_reduce(const float *partials, int parts, int ntiles, int mt, int bn, int M, int N, void *C, int c_f32,
                                  int accumulate, hipStream_t st) {
-    if (parts < 2 || parts > 4 || mt < 1 || ntiles < 1) return hipErrorInvalidValue;
+    if (parts < 2 || parts > HQ_WR8_PARTS || (bn != 192 && parts > 4) || mt < 1 || ntiles < 1) return hipErrorInvalidValue;
     const unsigned grid = (unsigned)(((size_t)ntiles * WR_BM * (bn / 8) + 255) / 256);
-    if (bn == 160) k_tile_reduce<160><<<grid, 256, 0, st>>>(partials, parts, ntiles, mt, M, N, C, c_f32, accumulate);
-    else if (bn == 192) k_tile_reduce<192><<<grid, 256, 0, st>>>(partials, parts, ntiles, mt, M, N, C, c_f32, accumulate);
+    if (bn == 160) k_tile_reduce<160, 4><<<grid, 256, 0, st>>>(partials, parts, ntiles, mt, M, N, C, c_f32, accumulate);
+    else if (bn == 192 && parts > 4) k_tile_reduce<192, HQ_WR8_PARTS><<<grid, 256, 0, st>>>(partials, parts, ntiles, mt, M, N, C, c_f32, accumulate);
+    else if (bn == 192) k_tile_reduce<192, 4><<<grid, 256, 0, st>>>(partials, parts, ntiles, mt, M, N, C, c_f32, accumulate);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }

@@ -52,6 +52,8 @@ struct Wr8Args {
     void *C;
     int c_f32, accumulate;
     int mt, nt0, nt;  // M-tiles; this launch's column tiles nt0 .. nt - 1
+    int parts;        // workgroups per tile (K split)
+    float *partials;  // with parts > 1: [tile][part] fp32 tiles in tile_finish's layout
 };
 
 struct Wr8Lds {
@@ -130,17 +132,40 @@ DEV void w8_grp_dec(f4 &c0, f4 &c1, f4 &c2, const u4v &b0, const u4v &b1, const 
 // the latency of the last MFMAs before their accumulators are read by other instructions
 DEV void w8_mfma_drain() { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory"); }
 
-__global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr(Wr8Args g) {
+// A part's fp32 tile from LDS (rows of W8_LD floats) to its place in the workspace, in the order that
+// k_tile_reduce reads (tile_finish's); rows past M are left out, nothing reads them.
+constexpr int W8_LD = Wr8Lds::BN + 4;
+DEV void w8_store_part(const char *lds, const Wr8Args &g, int tile, int part, int rows, int tid) {
+    constexpr int CH = Wr8Lds::BN / 8, NCH = W8_BM * CH;
+    constexpr uint32_t TILE = W8_BM * Wr8Lds::BN * 4;
+    static_assert(W8_BM * W8_LD * 4 <= Wr8Lds::TOTAL, "fp32 tile in LDS");
+    const rsrc_t rp = make_rsrc(g.partials, (uint32_t)g.mt * (uint32_t)g.nt * (uint32_t)g.parts * TILE);
+    const uint32_t own = ((uint32_t)tile * (uint32_t)g.parts + (uint32_t)part) * TILE;
+    for (int c = tid; c < CH * rows; c += W8_NT) {
+        const int row = c / CH, ch = c - row * CH;
+        const char *p = lds + (row * W8_LD + 8 * ch) * 4;
+        buf_store16(rp, *(const f4 *)p, own + (uint32_t)c * 16u);
+        buf_store16(rp, *(const f4 *)(p + 16), own + (uint32_t)(c + NCH) * 16u);
+    }
+}
+
+// KS: with the K split (compiled out of the whole-K kernel)
+template <bool KS>
+DEV void w8_tile(const Wr8Args &g) {
     using L = Wr8Lds;
     constexpr int NB = W8_NB, BN = L::BN, WC = L::WC;
     __shared__ __attribute__((aligned(256))) char lds[L::TOTAL];
     // tile: XCD x = b % 8 takes N-tiles x, x + 8, ...; its slots run over the M-tiles of one N-tile
     // first (the weight slab is then fetched once per XCD)
     const int b = blockIdx.x, x = b & 7, j8 = b >> 3;
-    const int nt_i = g.nt0 + x + 8 * (j8 / g.mt), mt_i = j8 % g.mt;
+    // K split: the same over (N-tile, part) pairs
+    const int parts = KS ? g.parts : 1, cu = x + 8 * (j8 / g.mt);
+    const int nt_i = KS ? cu / parts : g.nt0 + cu, part = KS ? cu - nt_i * parts : 0, mt_i = j8 % g.mt;
     if (nt_i >= g.nt) return;
     const int m0 = mt_i * W8_BM, n0 = nt_i * BN;
-    const int M = g.M, N = g.N, K = g.K, U = K / 256, S2 = 4 * U;
+    const int M = g.M, N = g.N, K = g.K, Ut = K / 256;
+    // this workgroup's super-stages u0 .. u0 + U - 1 (u and s below count from u0)
+    const int u0 = KS ? part * Ut / parts : 0, U = KS ? (part + 1) * Ut / parts - u0 : Ut, S2 = 4 * U;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 15,
               lg = lane >> 4;
     // roles: waves 0-3 multiply (wave w: columns 48w .. 48w + 47 of the tile, all 128 rows); waves 4-7
@@ -180,16 +205,16 @@ __global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr(Wr8Args g) {
 #pragma unroll
             for (int q = 0; q < 4; q++)
                 dma16_so(ra, lds0 + (uint32_t)(L::A + buf * L::A_BYTES + w4 * 4096 + q * 1024), a_voff[q],
-                         (uint32_t)(s * W8_KS * 2));
+                         (uint32_t)((4 * u0 + s) * W8_KS * 2));
         };
         auto dma_q = [&](int s, int buf) {
 #pragma unroll
             for (int t = 0; t < 3; t++)
                 dma16_so(rq, lds0 + (uint32_t)(L::Q + buf * L::Q_BYTES + (w4 + 4 * t) * 1024), q_voff[t],
-                         (uint32_t)(s * W8_KS));
+                         (uint32_t)((4 * u0 + s) * W8_KS));
         };
         auto dma_d = [&](int v) {
-            dma16_so(rd, lds0 + (uint32_t)(L::D + (v & 1) * L::D_BYTES + w4 * 1024), d_voff, (uint32_t)(16 * v));
+            dma16_so(rd, lds0 + (uint32_t)(L::D + (v & 1) * L::D_BYTES + w4 * 1024), d_voff, (uint32_t)(16 * (u0 + v)));
         };
         // prologue: stage 0 and the scales of super-stage 0, then stage 1 (still in flight at the
         // barrier, as every loader stage's loads are)
@@ -222,12 +247,13 @@ __global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr(Wr8Args g) {
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last (clamped, unused) loads
-        if (tile_store_ok(g.c_f32, g.accumulate, g.N, g.C)) {
+        if (KS || tile_store_ok(g.c_f32, g.accumulate, g.N, g.C)) {
             // meet the MFMA waves once they are done with the rings and once their tile is in LDS,
             // then store it with them
             w8_barrier();
             w8_barrier();
-            w8_store(lds, g, m0, n0, tid);
+            if constexpr (KS) w8_store_part(lds, g, nt_i * g.mt + mt_i, part, min(W8_BM, M - m0), tid);
+            else w8_store(lds, g, m0, n0, tid);
         }
         return;
     }
@@ -322,6 +348,17 @@ __global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr(Wr8Args g) {
         }
     }
     w8_mfma_drain();
+    if constexpr (KS) {
+        w8_barrier();  // every wave is done with the rings and scales
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) *(f4 *)(lds + ((16 * i + ln) * W8_LD + wc0 + 16 * j + 4 * lg) * 4) = acc[i][j];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        w8_barrier();
+        w8_store_part(lds, g, nt_i * g.mt + mt_i, part, min(W8_BM, M - m0), tid);
+        return;
+    }
     // fp16 C through LDS (tile_store_rows) where C allows it: the accumulators as fp16 at their rows
     // and columns, then all 8 waves store
     if (tile_store_ok(g.c_f32, g.accumulate, g.N, g.C)) {
@@ -401,6 +438,14 @@ __global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr(Wr8Args g) {
         }
     }
 }
+
+__global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr(Wr8Args g) { w8_tile<false>(g); }
+// Each tile's K split over `parts` workgroups; k_tile_reduce adds their tiles. For few tiles over a long K: whole-K
+// tiles leave CUs idle, and the LDS-decode kernel's split (two waves' decode and its ring of 128-k stages) runs at
+// half this loop's rate. A 256-wide super-stage takes 1.6 us with few workgroups, 2.1 with 224 (L2); launches,
+// prologue, parts' round trip and sum 9 us + 0.23 us per MB of parts. M = 384, N = 4096, K = 15360: 96 -> 57 us
+// (839 TFLOP/s); M = 512, N = 2560, K = 9728: 37.5 -> 34 (750); M = 128: 26.3 -> 19.5 (327).
+__global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr_ks(Wr8Args g) { w8_tile<true>(g); }
 }  // namespace
 
 // every byte offset of the kernel (tile rows and columns past the matrix included, C's) fits 32 bits
@@ -411,7 +456,7 @@ int hq_wr8_fits(const hq_dev_mat *W, int M) {
 }
 
 hipError_t hq_launch_gemm_wr8(const hq_dev_mat *W, const uint16_t *A, int M, void *C, int c_f32, int accumulate,
-                              int nt0, int nt1, hipStream_t st) {
+                              int nt0, int nt1, int parts, float *partials, hipStream_t st) {
     if (!hq_wr8_fits(W, M)) return hipErrorInvalidValue;
     // fp32 or fp16 C, or the SwiGLU output of a gate/up pair matrix (N a multiple of 16, no accumulate)
     if (c_f32 != 0 && c_f32 != 1 && !(c_f32 == HQ_OUT_SWIGLU && W->rows % 16 == 0 && !accumulate)) return hipErrorInvalidValue;
@@ -422,7 +467,17 @@ hipError_t hq_launch_gemm_wr8(const hq_dev_mat *W, const uint16_t *A, int M, voi
     const int nt_all = (g.N + 64 * W8_NB - 1) / (64 * W8_NB);
     g.nt0 = nt0, g.nt = nt1 < 0 || nt1 > nt_all ? nt_all : nt1;
     if (nt0 < 0 || nt0 >= g.nt) return hipErrorInvalidValue;
-    const unsigned grid = (unsigned)(8 * ((g.nt - g.nt0 + 7) / 8) * g.mt);
+    // K split: whole super-stages per part, all columns, a workspace of one fp32 tile per (tile, part), 32-bit offsets
+    g.parts = parts, g.partials = partials;
+    if (parts < 1 || parts > HQ_WR8_PARTS || parts > g.K / 256) return hipErrorInvalidValue;
+    if (parts > 1 && (!partials || nt0 != 0 || g.nt != nt_all || c_f32 == HQ_OUT_SWIGLU ||
+                      (size_t)g.mt * g.nt * parts * W8_BM * 64 * W8_NB * 4 >= ((size_t)1 << 32)))
+        return hipErrorInvalidValue;
+    const unsigned grid = (unsigned)(8 * (((g.nt - g.nt0) * parts + 7) / 8) * g.mt);
+    if (parts > 1) {
+        k_gemm_q8_0_wr_ks<<<grid, W8_NT, 0, st>>>(g);
+        return hq_launch_tile_reduce(partials, parts, g.mt * g.nt, g.mt, 64 * W8_NB, M, g.N, C, c_f32, accumulate, st);
+    }
     k_gemm_q8_0_wr<<<grid, W8_NT, 0, st>>>(g);
     return hipGetLastError();
 }

@@ -95,10 +95,12 @@ hipError_t hq_launch_tile_reduce(const float *partials, int parts, int ntiles, i
                                  int accumulate, hipStream_t st);
 hipError_t hq_launch_gemm_wr(const hq_dev_mat *W, const uint16_t *A, int M, void *C, int c_f32, int accumulate,
                              int nt0, int nt1, int parts, float *partials, int *counters, hipStream_t st, int tw = 192);
-// The same tile shape for Q8_0 (hq_gemm_wr8.hip; K a multiple of 256, no workspace).
+// The same tile shape for Q8_0 (hq_gemm_wr8.hip; K a multiple of 256). With parts > 1 each tile's K
+// is split over that many workgroups (every column tile, no SwiGLU) and partials holds a tile per part.
+constexpr int HQ_WR8_PARTS = 8;  // most parts; k_tile_reduce's too (192-column tiles)
 int hq_wr8_fits(const hq_dev_mat *W, int M);
 hipError_t hq_launch_gemm_wr8(const hq_dev_mat *W, const uint16_t *A, int M, void *C, int c_f32, int accumulate,
-                              int nt0, int nt1, hipStream_t st);
+                              int nt0, int nt1, int parts, float *partials, hipStream_t st);
 // Mid-M Q4_K GEMM (hq_gemm_rb.hip): whether M, K suit it (33 <= M <= 64, K a multiple of 512,
 // 32-bit offsets), its workgroups per tile for a shape, and the launch (no pre-pass: the kernel forms
 // the activation sub-block sums; partials / counters as for the other K splits when parts > 1).

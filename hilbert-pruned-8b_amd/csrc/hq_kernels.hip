@@ -1040,6 +1040,7 @@ struct GemmCfg {
     int wr_tw;      // with wr: tile width, 192 or 160 columns (k_gemm_q4_k_wr160)
     bool wr_multi;  // with wr: launches of at most one round each (wr4_plan), no K split
     bool wr8;       // Q8_0, the same: k_gemm_q8_0_wr (hq_gemm_wr8.hip)
+    int wr8_parts;  // with wr8: workgroups per tile (K split), 1: whole K
     bool nn;        // Q4_K with N <= 32 and many rows: k_gemm_q4_k_nn (hq_gemm_nn.hip)
     HqSmPlan sm;    // sm.parts > 0: few output tiles, the small-tile kernels of hq_gemm_sm.hip
 };
@@ -1053,6 +1054,19 @@ float ws_us(int type, int M, int N, int K, int nb, int parts, int n_cu) {
     const long wgs = (long)((M + 127) / 128) * ((N + 32 * nb - 1) / (32 * nb)) * parts, rounds = (wgs + n_cu - 1) / n_cu;
     const float stages = (float)(rounds * ((K / 128 + parts - 1) / parts));
     return f.base + stages * (f.stage + f.stage_nb * nb) + (parts > 1 ? f.split * nb * parts : 0.f) + f.round * (float)(rounds - 1);
+}
+
+// Parts of K for k_gemm_q8_0_wr_ks with the least estimated us, one round on every XCD: launches, prologue,
+// epilogue and the sum's launch; 256-wide super-stages, slower the more workgroups share L2; the parts' bytes
+// (fit over N = 1024 .. 19456, K = 1024 .. 15360, M = 65 .. 1024: most within 7 %). 0: none fits.
+int wr8_split(int M, int N, int K, int n_cu, float *us) {
+    const int mt = (M + 127) / 128, nt = (N + 191) / 192, U = K / 256;
+    int best = 0;
+    for (int p = 2; p <= std::min(U, HQ_WR8_PARTS) && mt * ((nt * p + 7) / 8) <= n_cu / 8; p++) {
+        const float t = 9.2f + (1.6f + .002f * (float)(mt * nt * p)) * (float)((U + p - 1) / p) + .92e-6f * (float)p * (float)M * (float)N;
+        if (!best || t < *us) best = p, *us = t;
+    }
+    return best;
 }
 
 // Whether the small-tile kernels (plan p) run instead of the kernel that c names so far. They replaced the
@@ -1209,6 +1223,25 @@ GemmCfg gemm_cfg(const hq_dev_mat *W, int M, int n_cu) {
     // at most one round each fill at least 70 % of the CU time (M = 512, N = 9728: one launch of 204
     // tiles; M = 2048: four launches of 16 x 13 tiles)
     c.wr8 = W->type == HQ_TYPE_Q8_0 && M > 64 && hq_wr8_fits(W, M) && wr_plan(M, (int)W->rows, n_cu).fill;
+    c.wr8_parts = 1;
+    // otherwise the same kernel with each tile's K split over 2 .. 8 workgroups in one round, by the estimates: for
+    // K >= 6144 wherever it is the faster (M = 128, N = 2560, K = 9728: small tiles 26.3 -> 19.5 us; M = 301: LDS-decode
+    // tiles 34.5 -> 27.7; M = 700: 64.6 -> 50.4; M = 301, N = 4096, K = 11008: 71.8 -> 42.0; 80 shapes from K = 6144 to
+    // 15360, M = 65 .. 1500: all faster, 1.04 to 2.2x). For a shorter K only over one row tile in 2 or 3 parts (M = 65,
+    // N = 15360, K = 4096: 32.4 -> 24.0; M = 128, N = 19456, K = 2560: 25.9 -> 24.3): with more row tiles or parts
+    // their sum takes what the split saves (M = 128, N = 9728, K = 2560: 16.6 against 17.9; M = 512, N = 2560,
+    // K = 4096: 21.7 against 21.4 at best). Not where the LDS-decode kernel's own split fills 80 % of the chip with rows
+    // and columns that exist, the shapes that tests hold it to, where least is to be had (M = 512, N = 2560,
+    // K = 9728: 37.5 against 34; M = 256: 25.9 against 23.1).
+    if (!c.wr8 && W->type == HQ_TYPE_Q8_0 && M > 64 && hq_wr8_fits(W, M)) {
+        const int N = (int)W->rows, K = (int)W->cols;
+        float us = 0.f;
+        const int parts = wr8_split(M, N, K, n_cu, &us);
+        const float now = c.ws8_nb ? ws_us(W->type, M, N, K, c.ws8_nb, c.ws8_parts, n_cu) : hq_sm_plan(W, M, n_cu).us;
+        const bool full = c.ws8_parts > 1 && 5L * M * N * c.ws8_parts >= 4L * n_cu * 128 * 32 * c.ws8_nb;
+        if (parts > 1 && !full && (K >= 6144 ? us < now : M <= 128 && parts <= 3 && c.ws8_nb && us < .95f * now))
+            c.wr8 = true, c.wr8_parts = parts;
+    }
     // N <= 32 with at least 64 workgroups of 64 rows (config 4's b / a projections at M = 16384: 256):
     // the skinny kernel, which reads A once with every CU streaming
     c.nn = W->type == HQ_TYPE_Q4_K && W->rows <= 32 && M >= 64 * 64 && hq_nn_fits(W, M);
@@ -1298,7 +1331,7 @@ void hq_gemm_kernel_name(int type, int M, int N, int K, int n_cu, char *buf, siz
     else if (c.wr)
         snprintf(buf, n, c.wr_parts > 1 ? (c.wr_tw == 160 ? "k_gemm_q4_k_wr_ks160" : "k_gemm_q4_k_wr_ks<3>")
                                         : c.wr_tw == 160 ? "k_gemm_q4_k_wr160" : "k_gemm_q4_k_wr<3>");
-    else if (c.wr8) snprintf(buf, n, "k_gemm_q8_0_wr");
+    else if (c.wr8) snprintf(buf, n, c.wr8_parts > 1 ? "k_gemm_q8_0_wr_ks" : "k_gemm_q8_0_wr");
     else if (c.ws_nb) snprintf(buf, n, "k_gemm_q4_k_ws<%d>", c.ws_nb);
     else if (c.ws8_nb) snprintf(buf, n, "k_gemm_q8_0_ws<%d>", c.ws8_nb);
     else snprintf(buf, n, "k_gemm_q4_k_w<8>");  // template argument: row blocks
@@ -1337,7 +1370,11 @@ void hq_gemm_work_bytes(const hq_dev_mat *W, int M, int n_cu, size_t *partial_by
     }
     // (the Q4_K tile kernels wr, ws form their own)
     *sums_bytes = c.wide && !c.wr && !(c.ws_nb && W->type == HQ_TYPE_Q4_K) ? (size_t)M * (W->cols / KC) * 32 : 0;
-    if (c.wr8) *partial_bytes = *counter_bytes = 0;  // (no K split)
+    if (c.wr8) {  // K split: one fp32 128 x 192 tile per (tile, part)
+        const size_t tiles = (size_t)((M + 127) / 128) * ((W->rows + 191) / 192);
+        *partial_bytes = c.wr8_parts > 1 ? tiles * c.wr8_parts * 128 * 192 * sizeof(float) : 0;
+        *counter_bytes = 0;
+    }
     if (c.wr) {  // K split: one fp32 128 x wr_tw tile per (tile, part)
         const size_t tiles = (size_t)((M + 127) / 128) * ((W->rows + c.wr_tw - 1) / c.wr_tw);
         *partial_bytes = c.wr_parts > 1 ? tiles * c.wr_parts * 128 * c.wr_tw * sizeof(float) : 0;
@@ -1377,10 +1414,11 @@ hipError_t hq_launch_gemm_main(const hq_dev_mat *W, const uint16_t *A, int M, vo
         });
     }
     if (c.wr) return hq_launch_gemm_wr(W, A, M, C, c_f32, accumulate, 0, -1, c.wr_parts, wk.partials, wk.counters, st, c.wr_tw);
+    if (c.wr8 && c.wr8_parts > 1) return hq_launch_gemm_wr8(W, A, M, C, c_f32, accumulate, 0, -1, c.wr8_parts, wk.partials, st);
     if (c.wr8) {
         const size_t K = W->cols, N = W->rows, esize = c_f32 ? 4 : 2;
         return wr_launches(wr_plan(M, (int)N, wk.n_cu), M, (int)N, [&](int m0, int rows, int t0, int t1) {
-            return hq_launch_gemm_wr8(W, A + (size_t)m0 * K, rows, (char *)C + (size_t)m0 * N * esize, c_f32, accumulate, t0, t1, st);
+            return hq_launch_gemm_wr8(W, A + (size_t)m0 * K, rows, (char *)C + (size_t)m0 * N * esize, c_f32, accumulate, t0, t1, 1, nullptr, st);
         });
     }
     if (c.ws_nb)
@@ -1440,7 +1478,7 @@ hipError_t hq_launch_gemm_swiglu(const hq_dev_mat *W, const uint16_t *A, int M, 
         return wr_launches(pl, M, N, [&](int m0, int rows, int t0, int t1) {
             const uint16_t *Am = A + (size_t)m0 * K;
             uint16_t *om = out + (size_t)m0 * (N / 2);
-            return wr8 ? hq_launch_gemm_wr8(W, Am, rows, om, HQ_OUT_SWIGLU, 0, t0, t1, st)
+            return wr8 ? hq_launch_gemm_wr8(W, Am, rows, om, HQ_OUT_SWIGLU, 0, t0, t1, 1, nullptr, st)
                        : hq_launch_gemm_wr(W, Am, rows, om, HQ_OUT_SWIGLU, 0, t0, t1, 1, nullptr, nullptr, st, pl.tw);
         });
     }

@@ -172,3 +172,36 @@ def test_wr8_several_launches(hqlib, oracle, M, N, K):
     rows = sample_rows(M, per_tile=4)
     ref = oracle.matmul(blocks, synth.Q8_0, N, K, oracle.f16_to_f32(a[rows]))
     check(got[rows], ref, f"wr8 launches ({len(rows)} rows)")
+
+
+@pytest.mark.parametrize("M,N,K", [(100, 2500, 6144), (500, 1030, 6400), (384, 2500, 6144), (768, 2498, 6144), (65, 15361, 4096)])
+def test_wr8_k_split(hqlib, oracle, M, N, K):
+    """k_gemm_q8_0_wr_ks and its sum: 2 to 8 parts of equal and unequal numbers of super-stages, ragged
+    last row and column tiles, N not a multiple of 8 (element-wise stores), every output mode. Bars: the
+    file's, and the operand rounding's bound against the float64 product (the parts' fp32 sums add at most 8
+    roundings of 2^-24 to it); the same bits from a second call."""
+    blocks = special_q8_0_weights(61 + N, N, K) if N < 15000 else synth.random_blocks(synth.Q8_0, synth.Rng(61), N, K)
+    a = synth.activations_f16(synth.Rng(62 + M), M, K)
+    name = hqlib.gemm_kernel(synth.Q8_0, M, N, K)
+    say(f"K split M={M} N={N} K={K} kernel={name}")
+    assert name == "k_gemm_q8_0_wr_ks"
+    W = hqlib.Mat(blocks, synth.Q8_0, N, K)
+    got = hqlib.gemm_np(W, a)
+    assert np.array_equal(got, hqlib.gemm_np(W, a))
+    c0 = synth.activations_f16(synth.Rng(63), M, N)
+    acc = hqlib.gemm_np(W, a, c_f32=True, c_init=c0.view(np.float16).astype(np.float32))
+    half = hqlib.gemm_np(W, a, c_f32=False).view(np.float16).astype(np.float64)
+    W.free()
+    rows = np.unique(np.r_[0:3, M // 128 * 128 - 1:M, M - 1])
+    cols = np.unique(np.r_[0:200, N // 192 * 192 - 1:N])
+    x = oracle.f16_to_f32(a[rows]).astype(np.float64)
+    w = oracle.dequantize(blocks, synth.Q8_0, N, K)[cols].astype(np.float64)
+    ref, bound = x @ w.T, np.abs(x) @ np.abs(w.T)
+    at = np.ix_(rows, cols)
+    assert np.all(np.abs(got[at] - ref) <= OPERAND_BOUND * bound)
+    c = c0.view(np.float16).astype(np.float64)[at]
+    assert np.all(np.abs(acc[at] - (ref + c)) <= OPERAND_BOUND * bound + 2.0 ** -24 * np.abs(c))
+    # fp16 outputs: one rounding more, where the value lies in fp16's range (these scales give some beyond 65504)
+    fits = np.abs(ref) + OPERAND_BOUND * bound < 65504
+    assert fits.mean() > 0.5
+    assert np.all((np.abs(half[at] - ref) <= OPERAND_BOUND * bound * (1 + 2.0 ** -11) + 2.0 ** -11 * np.abs(ref) + 2.0 ** -25)[fits])
