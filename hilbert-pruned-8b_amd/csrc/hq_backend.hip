@@ -4,7 +4,7 @@
 // Per chunk of T tokens at position pos0 (the reference's run_layers, src/cuda_backend.cu:783-850,
 // for LAYER_FULL layers), on the backend's stream:
 //   x [T, H] fp32      residual stream (embedding rows decoded from the GGUF blocks)
-//   hb [T, H] fp16     RMSNorm(x) * (off + w): the GEMM operand (k_rmsnorm_f16)
+//   hb [T, H] fp16     RMSNorm(x) * (off + w): the GEMM operand (k_rmsnorm; for one token inside the GEMV, hq_launch_gemv_norm)
 //   q/k/v fp32         hq_gemm(q|k|v, hb)            (q rows interleave [q_h | gate_h] with the output gate);
 //        of one block type they are resident as one matrix, and one hq_gemm fills rows [q | k | v]
 //   qr fp32, kc/vc     q/k RMSNorm (optional) + RoPE with the model's inverse frequencies, k and v
@@ -373,12 +373,17 @@ int run_layers(HipBackend *b, int T, int pos0) {
     hipStream_t st = b->st;
     for (uint32_t li = 0; li < c.n_layers; li++) {
         const DevLayer &L = b->L[li];
-        k_rmsnorm<_Float16><<<T, 256, 0, st>>>(b->x, L.in_norm, off, eps, b->hb, H);
-        BCK(hipGetLastError());
+        // one token: the norm inside the GEMV where it has such a kernel
+        int fused = 0;
+        if (T == 1 && L.qkv) BCK(hq_launch_gemv_norm(hq_mat_dev(L.qkv), b->x, L.in_norm, off, eps, 0, b->qb, st, &fused));
+        if (!fused) {
+            k_rmsnorm<_Float16><<<T, 256, 0, st>>>(b->x, L.in_norm, off, eps, b->hb, H);
+            BCK(hipGetLastError());
+        }
         const float *kb = b->kb, *vb = b->vb;
         int sq = qw, skv = nkv * hd;
         if (L.qkv) {
-            if (gemm(b, L.qkv, b->hb, T, b->qb, false)) return -1;
+            if (!fused && gemm(b, L.qkv, b->hb, T, b->qb, false)) return -1;
             kb = b->qb + qw, vb = kb + skv;
             sq = skv = qw + 2 * skv;
         } else if (gemm(b, L.q, b->hb, T, b->qb, false) || gemm(b, L.k, b->hb, T, b->kb, false) ||
@@ -394,10 +399,14 @@ int run_layers(HipBackend *b, int T, int pos0) {
         const HqAttnArgs at = {b->qr, b->qb, L.kc, L.vc, b->ob, b->att_part, b->att_cnt, T, nh, nkv, hd, sq, c.attn_gate, pos0, scale};
         BCK(hq_launch_attention(at, b->n_cu, st));
         if (gemm(b, L.o, b->ob, T, b->x, true)) return -1;
-        k_rmsnorm<_Float16><<<T, 256, 0, st>>>(b->x, L.post_norm, off, eps, b->hb, H);
-        BCK(hipGetLastError());
+        fused = 0;
+        if (T == 1 && L.pair) BCK(hq_launch_gemv_norm(hq_mat_dev(L.pair), b->x, L.post_norm, off, eps, 1, b->fb, st, &fused));
+        if (!fused) {
+            k_rmsnorm<_Float16><<<T, 256, 0, st>>>(b->x, L.post_norm, off, eps, b->hb, H);
+            BCK(hipGetLastError());
+        }
         if (L.pair) {
-            if (hq_gemm_swiglu(L.pair, (const uint16_t *)b->hb, T, (uint16_t *)b->fb, st)) return -1;
+            if (!fused && hq_gemm_swiglu(L.pair, (const uint16_t *)b->hb, T, (uint16_t *)b->fb, st)) return -1;
         } else if (T == 1) {
             k_gateup_swiglu<<<(I + 3) / 4, 256, 0, st>>>(*hq_mat_dev(L.gate), *hq_mat_dev(L.up), b->hb, b->fb, I, H);
             BCK(hipGetLastError());

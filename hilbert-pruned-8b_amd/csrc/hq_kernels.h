@@ -38,6 +38,10 @@ hipError_t hq_launch_gemv(const hq_dev_mat *W, const uint16_t *a, void *C, int c
 // M = 1 of a gate/up pair matrix: out[i] = fp16(silu(gate_i . a) * (up_i . a)), the GEMV kernels' dots and
 // the product in their epilogue (*fused = 0: no such kernel for the shape, nothing was launched)
 hipError_t hq_launch_gemv_pair(const hq_dev_mat *W, const uint16_t *a, uint16_t *out, hipStream_t st, int *fused);
+// M = 1 with a = fp16(RMSNorm(x) * (off + w)) of fp32 x [K]: fp32 W . a, or of a gate/up pair matrix the SwiGLU
+// as above (*fused = 0: nothing was launched)
+hipError_t hq_launch_gemv_norm(const hq_dev_mat *W, const float *x, const float *w, float off, float eps, int pair, void *out,
+                               hipStream_t st, int *fused);
 // Stream-K workspace: fp32 partial tiles and per-tile counters (zero when idle; each launch leaves
 // them zero), the activation sub-block sums of the wide Q4_K kernel, and the number of CUs the
 // persistent grid is sized for.

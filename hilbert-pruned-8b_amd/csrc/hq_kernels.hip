@@ -194,12 +194,26 @@ DEV float dot_row_q4_k(const uint8_t *__restrict__ row, const uint16_t *__restri
 // slice into registers and reused by the R rows, all R x TS weight loads of a slice in flight together.
 constexpr int GV_TS = 2;  // 16-byte chunks per lane per K slice
 
+// 16 quants (bytes q + 128) of a Q8_0 row times their activations
+DEV float chunk_q8_0(const u4v q, const u4v a0, const u4v a1) {
+    const h2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+    h2 lo[4], hi[4];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        lo[2 * i] = as_h2(perm_lo(w[i])) + bias;
+        lo[2 * i + 1] = as_h2(perm_hi(w[i])) + bias;
+        hi[2 * i] = as_h2(perm_lo(w[2 + i])) + bias;
+        hi[2 * i + 1] = as_h2(perm_hi(w[2 + i])) + bias;
+    }
+    return dot8(hi, a1, dot8(lo, a0, 0.f));
+}
+
 // Q8_0: R rows n0 .. n0+R-1 (clamped) against activation vector a; returns the lane's partials.
 template <int R>
 DEV void rows_q8_0(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ d, int ldd,
                    const uint16_t *__restrict__ a, int K, const int (&n)[R], int j, float (&acc)[R]) {
     const int nch = K / 16;
-    const h2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
 #pragma unroll
     for (int r = 0; r < R; r++) acc[r] = 0.f;
     for (int c0 = j; c0 < nch; c0 += 64 * GV_TS) {
@@ -220,17 +234,50 @@ DEV void rows_q8_0(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ 
         for (int t = 0; t < GV_TS; t++)
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                const uint32_t w[4] = {q[r][t].x, q[r][t].y, q[r][t].z, q[r][t].w};
-                h2 lo[4], hi[4];
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    lo[2 * i] = as_h2(perm_lo(w[i])) + bias;
-                    lo[2 * i + 1] = as_h2(perm_hi(w[i])) + bias;
-                    hi[2 * i] = as_h2(perm_lo(w[2 + i])) + bias;
-                    hi[2 * i + 1] = as_h2(perm_hi(w[2 + i])) + bias;
-                }
-                acc[r] += dot8(hi, a1[t], dot8(lo, a0[t], 0.f)) * dv[r][t];
+                acc[r] += chunk_q8_0(q[r][t], a0[t], a1[t]) * dv[r][t];
             }
+    }
+}
+
+// The same with a = fp16(RMSNorm(x) * (off + w)) formed by the wave itself (the arithmetic of k_rmsnorm): lane j
+// has the values of its own NT chunks in registers, so the sum of squares takes one wave reduction and
+// nothing is staged; the weights are on their way meanwhile. K <= 1024 NT.
+template <int R, int NT>
+DEV void rows_q8_0_norm(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ d, int ldd, const float *__restrict__ x,
+                        const float *__restrict__ w, float off, float eps, int K, const int (&n)[R], int j, float (&acc)[R]) {
+    const int nch = K / 16;
+    f4 xv[NT][4], wv[NT][4];
+    u4v q[R][NT];
+    float dv[R][NT], ss = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int c = j + 64 * t, cc = c < nch ? c : nch - 1;
+#pragma unroll
+        for (int i = 0; i < 4; i++) xv[t][i] = *(const f4 *)(x + 16 * cc + 4 * i), wv[t][i] = *(const f4 *)(w + 16 * cc + 4 * i);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            q[r][t] = load16(qs + (size_t)n[r] * K + 16 * cc);
+            dv[r][t] = c < nch ? h2f(d[(size_t)n[r] * ldd + (cc >> 1)]) : 0.f;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+        if (j + 64 * t < nch)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) ss += xv[t][i][e] * xv[t][i][e];
+    const float inv = 1.0f / sqrtf(row_sum<64>(ss) / (float)K + eps);
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        h8 a[2];
+#pragma unroll
+        for (int i = 0; i < 16; i++) a[i >> 3][i & 7] = (_Float16)(xv[t][i >> 2][i & 3] * inv * (off + wv[t][i >> 2][i & 3]));
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            acc[r] += j + 64 * t < nch ? chunk_q8_0(q[r][t], __builtin_bit_cast(u4v, a[0]), __builtin_bit_cast(u4v, a[1])) * dv[r][t] : 0.f;
     }
 }
 
@@ -470,6 +517,26 @@ __global__ void __launch_bounds__(256) k_gemv_q8_0_pair(const uint8_t *__restric
     rows_q8_0<2>(qs, d, ldd, a, K, n, j, acc);
     const float g = row_sum<64>(acc[0]), u = row_sum<64>(acc[1]);
     if (j == 0) out[i] = swiglu_f16(g, u);
+}
+
+// Both with the RMSNorm of their input (rows_q8_0_norm): a wave per output row, or per gate/up pair
+template <int NT, bool PAIR>
+__global__ void __launch_bounds__(256) k_gemv_q8_0_norm(const uint8_t *__restrict__ qs, const uint16_t *__restrict__ d, int ldd,
+                                                        const float *__restrict__ x, const float *__restrict__ w, float off,
+                                                        float eps, int N, int K, void *__restrict__ out) {
+    constexpr int R = PAIR ? 2 : 1;
+    const int j = threadIdx.x & 63, i = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (i >= N / R) return;
+    int n[R];
+    n[0] = PAIR ? pair_row(i) : i;
+    if constexpr (PAIR) n[1] = n[0] + 8;
+    float acc[R];
+    rows_q8_0_norm<R, NT>(qs, d, ldd, x, w, off, eps, K, n, j, acc);
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = row_sum<64>(acc[r]);
+    if (j) return;
+    if constexpr (PAIR) ((uint16_t *)out)[i] = swiglu_f16(acc[0], acc[1]);
+    else ((float *)out)[i] = acc[0];
 }
 
 template <int R>
@@ -899,6 +966,28 @@ hipError_t hq_launch_gemv(const hq_dev_mat *W, const uint16_t *a, void *C, int c
     } else {
         launch_gemv_t<1>(W, a, C, c_f32, accumulate, st);
     }
+    return hipGetLastError();
+}
+
+// The norm inside the GEMV saves a launch of 2.8 us and the gap before it. Every wave then reads all of x and w (8 K
+// bytes, from L2): at 16 MB for all waves about 2 us, so more than that, or more than two chunks of registers a
+// lane, leaves the norm its own launch. A token of the 4-layer, 512-wide Llama behind 1000: 166 -> 138 us.
+constexpr size_t NORM_BYTES = (size_t)16 << 20;
+hipError_t hq_launch_gemv_norm(const hq_dev_mat *W, const float *x, const float *w, float off, float eps, int pair, void *out,
+                               hipStream_t st, int *fused) {
+    const int N = (int)W->rows, K = (int)W->cols, waves = pair ? N / 2 : N;
+    *fused = W->type == HQ_TYPE_Q8_0 && K <= 2048 && (size_t)waves * K * 8 <= NORM_BYTES && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    if (!*fused) return hipSuccess;
+    const unsigned grid = (unsigned)((waves + 3) / 4);
+#define GN(nt, p) k_gemv_q8_0_norm<nt, p><<<grid, 256, 0, st>>>(W->qs, W->d, W->ldd, x, w, off, eps, N, K, out)
+    if (K <= 1024) {
+        if (pair) GN(1, true);
+        else GN(1, false);
+    } else {
+        if (pair) GN(2, true);
+        else GN(2, false);
+    }
+#undef GN
     return hipGetLastError();
 }
 

@@ -73,3 +73,28 @@ def test_passes_of_a_long_prompt(hqlib, oracle, nh, nkv, rot, T):
     be.destroy()
     ref = oracle.llama_forward(model, tokens, ids)
     assert max_abs(got, ref) <= 1e-2 and max_abs(split, got) <= 1e-3
+
+
+@pytest.mark.parametrize("gtype,hidden,inter", [(synth.Q8_0, 256, 64), (synth.Q8_0, 1024, 288), (synth.Q8_0, 1056, 288), (synth.Q8_0, 2048, 256),
+                                                (synth.Q8_0, 2080, 256), (synth.Q8_0, 512, 8224)])
+def test_one_token_norm(hqlib, oracle, gtype, hidden, inter):
+    """One token's RMSNorm inside the q/k/v and gate/up GEMVs, on both sides of their rule (hidden up to 2048, waves
+    x hidden x 8 up to 16 MB) and of a lane's one or two chunks of 16 values, some lanes without one: the logits
+    of a one-token pass against the oracle's and against the same tokens in one pass, whose norm is the kernel of
+    its own."""
+    cfg = dict(synth.TINY_LLAMA, n_layers=2, hidden=hidden, intermediate=inter, vocab=512, n_heads=2, n_kv_heads=1, head_dim=32, rot_dim=32)
+    model = synth.tiny_llama(hidden, cfg)
+    tokens, ids = synth.tiny_llama_prompt(12, T=4, vocab=512, n_ids=16)
+    be = hqlib.HipBackend(hqlib.RefModelView(model), 4)
+    for t in range(3):
+        be.forward(tokens[t:t + 1])
+    one = be.forward(tokens[3:], ids)
+    be.reset()
+    whole = be.forward(tokens, ids)
+    be.destroy()
+    ref = oracle.llama_forward(model, tokens, ids)
+    print(f"[gpu] one-token norm H={hidden} I={inter}: max_abs {max_abs(one, ref):.2e}", flush=True)
+    # one against whole: fp16 roundings (2^-11 / sqrt(3) in the mean) of four GEMM inputs in each of two layers and of the
+    # whole pass's Q8_0 weights (the GEMVs' are exact), 24 in all, on logits of deviation 0.02 sqrt(2080) = 0.91:
+    # sqrt(24) 2.8e-4 0.91 = 1.3e-3, three of them
+    assert max_abs(one, ref) <= 1e-2 and max_abs(one, whole) <= 3.8e-3
