@@ -545,6 +545,7 @@ extern "C" int hq_dequant_f32(const hq_mat *W, uint32_t row0, uint32_t nrows, fl
 
 extern "C" int hq_gemm(const hq_mat *W, const uint16_t *A, int M, void *C, int c_is_f32, int accumulate, void *stream) {
     if (!W || !A || !C) return fail("hq_gemm: null argument");
+    c_is_f32 = c_is_f32 != 0;  // the launchers' other output mode (HQ_OUT_SWIGLU) is hq_gemm_swiglu's alone
     if (M < 1 || M > (1 << 23)) return fail("hq_gemm: M = %d (1 .. 8388608)", M);
     if (!aligned(A, 16)) return fail("hq_gemm: A must be 16-byte aligned");
     if (!aligned(C, c_is_f32 ? 4 : 2)) return fail("hq_gemm: C is misaligned");
@@ -644,6 +645,7 @@ extern "C" int hq_gemm_workspace_bytes(int ggml_type, int M, uint32_t N, uint32_
 extern "C" int hq_gemm_noalloc(const hq_mat *W, const uint16_t *A, int M, void *C, int c_is_f32, int accumulate,
                                void *stream) {
     if (!W || !A || !C) return fail("hq_gemm_noalloc: null argument");
+    c_is_f32 = c_is_f32 != 0;
     if (M < 1 || M > (1 << 23)) return fail("hq_gemm_noalloc: M = %d (1 .. 8388608)", M);
     if (!aligned(A, 16)) return fail("hq_gemm_noalloc: A must be 16-byte aligned");
     if (!aligned(C, c_is_f32 ? 4 : 2)) return fail("hq_gemm_noalloc: C is misaligned");
@@ -925,6 +927,7 @@ extern "C" int hq_time_gemm_kernel(hq_mat *const *Ws, int n_w, const uint16_t *A
                                    int iters, int reps, void *stream, float *ms) {
     if (!Ws || n_w < 1) return fail("hq_time_gemm_kernel: no matrices");
     if (M < 2) return fail("hq_time_gemm_kernel: M = %d (the GEMM kernels run for M >= 2)", M);
+    c_is_f32 = c_is_f32 != 0;
     for (int i = 0; i < n_w; i++)
         if (!Ws[i] || Ws[i]->m.rows != Ws[0]->m.rows || Ws[i]->m.cols != Ws[0]->m.cols || Ws[i]->m.type != Ws[0]->m.type)
             return fail("hq_time_gemm_kernel: matrices differ in shape or type");
