@@ -449,39 +449,43 @@ hipError_t hq_launch_gemm_sm(const hq_dev_mat *W, const uint16_t *A, int M, void
     case 11: SM_CASE(1, 1);
     case 21: SM_CASE(2, 1);
     case 41: SM_CASE(4, 1);
-    case 81:
-        if (W->type != HQ_TYPE_Q8_0) return hipErrorInvalidValue;
-        k_gemm_q8_0<8, 1><<<grid, SM_NT, 0, st>>>(g);
-        return hipGetLastError();
     default: return hipErrorInvalidValue;
     }
 #undef SM_CASE
 #undef SM_LAUNCH
 }
 
-// Rows per tile follow M. One super-block (K <= 256) leaves nothing to share: 128-column tiles. Above, the
-// workgroups per tile with the least estimated time, in us: launch, prologue and epilogue; the stages of
-// the fullest XCD's CUs, each the larger of its decode and products and of its share of the ~8.5 TB/s that
-// the LDS DMA moves from L2; and the partial tiles' round trip of a K split. (Measured over N, K = 512 ..
-// 9728 and M = 2 .. 1024: within 12 % at the 10th and 22 % at the 90th percentile.)
+// Rows per tile follow M. One super-block (K <= 256) leaves nothing to share: 128-column tiles (not for Q8_0, which other
+// kernels serve better there). Above, the row blocks and
+// workgroups per tile with the least estimated time. The estimate, in us: launch, prologue and epilogue; what each
+// further round of the fullest XCD costs; the stages of its CUs (decode and products, by type and rows); all stages'
+// MB through the LDS DMA; millions of outputs, dearer where rows of C are not whole 8-value pieces; and the partial tiles'
+// round trip of a K split. (Least squares over 51000 measured calls of every type, N = 1 .. 20000, K = 32 .. 15360,
+// M = 2 .. 8192: half within 4 %, nine in ten within 9 %, 18 % for K <= 256.)
 HqSmPlan hq_sm_plan(const hq_dev_mat *W, int M, int n_cu, int max_parts) {
     const int type = W->type, N = (int)W->rows, K = (int)W->cols, U = (K + 255) / 256;
-    if (U <= 1) {
-        const int mb = M <= 16 ? (type == HQ_TYPE_Q4_K ? 2 : 1) : M <= 32 ? 2 : M <= 64 || type != HQ_TYPE_Q8_0 ? 4 : 8;
-        return {mb, 1, 1, 0.f};
-    }
+    const bool q8 = type == HQ_TYPE_Q8_0, one = U <= 1;
+    struct Fit { float base, round, stage, read, out, ragged; };
+    static const Fit onek[3] = {{5.15f, 0.f, 0.f, .04f, 0.f, 12.2f}, {5.7f, 0.f, 0.f, 0.f, 0.f, 5.4f}, {7.f, 3.1f, 0.f, .06f, 0.f, 4.6f}},
+                     fit8[3] = {{4.65f, 0.f, .63f, .033f, 0.f, 14.3f}, {4.86f, 2.5f, .8f, .013f, 0.f, 3.6f}, {5.6f, 3.5f, .97f, .007f, .4f, 2.f}},
+                     fitk[3] = {{4.44f, 0.f, .4f, .033f, 0.f, 15.4f}, {4.84f, .8f, .5f, .022f, 0.f, 3.7f}, {5.47f, 3.8f, .7f, .02f, .53f, 2.7f}};
+    const float decode = one || q8 || type == HQ_TYPE_Q3_K ? 0.f : type == HQ_TYPE_Q6_K ? .26f : type == HQ_TYPE_Q5_K ? .155f : .04f;
+    const float q6 = one && type == HQ_TYPE_Q6_K ? 1.05f : 0.f, outputs = 1e-6f * (float)M * (float)N;
+    const int top = M <= 16 ? 0 : M <= 32 ? 1 : 2, low = !one && M > 64 ? 1 : top, cols = one ? 128 : 64;
+    const long nt = (N + cols - 1) / cols, xcd = std::max(1, n_cu / 8);
     HqSmPlan best = {0, 0, 0, 0.f};
-    const int mb1 = M <= 16 ? 1 : M <= 32 ? 2 : 4, mb0 = M > 64 ? 2 : mb1;
-    for (int mb = mb1; mb >= mb0; mb /= 2) {
-        const float busy = (mb == 1 ? .51f : mb == 2 ? .65f : .86f) * (type == HQ_TYPE_Q6_K ? 1.28f : 1.f);
-        const long nt = (N + 63) / 64, mt = (M + 16 * mb - 1) / (16 * mb), xcd = std::max(1, n_cu / 8);
-        const float bytes = (float)(16 * mb * 512 + 64 * 16 * sm_pitch(type));
+    for (int lg = top; lg >= low; lg--) {
+        const int mb = 1 << lg;
+        const Fit &f = one ? onek[lg] : q8 ? fit8[lg] : fitk[lg];
+        const long mt = (M + 16 * mb - 1) / (16 * mb);
+        const float bytes = 1e-6f * (float)(16 * mb * 512 + cols * 16 * sm_pitch(type));
         for (int parts = 1; parts <= std::min(max_parts, SM_PARTS) && (parts == 1 || (2 * parts <= U && mt * nt * parts <= n_cu)); parts++) {
             const long wgs = mt * nt * parts, rounds = nt < 8 ? (wgs + n_cu - 1) / n_cu : ((nt + 7) / 8 * mt * parts + xcd - 1) / xcd;
-            const float stage = std::max(busy, bytes * (float)std::min(wgs, (long)n_cu) * (1.f / 8.5e6f));
-            const float t = 3.9f + 2.f * (float)(rounds - 1) + (float)rounds * (float)((U + parts - 1) / parts) * stage +
-                            (parts > 1 ? 1.4f + .1f * parts + .25f * mb : 0.f);
-            if (!best.parts || t < best.us) best = {mb == 1 && type == HQ_TYPE_Q4_K ? 2 : mb, 2, parts, t};
+            const float stages = (float)((U + parts - 1) / parts);
+            const float t = f.base + q6 + std::max(f.round, decode > .1f ? 3.f : 0.f) * (float)(rounds - 1) + (float)rounds * stages * (f.stage + decode) +
+                            f.read * stages * (float)wgs * bytes + outputs * (f.out + (N % 8 ? f.ragged : 0.f)) +
+                            (parts > 1 ? 1.f + .19f * (float)parts + .13f * (float)mb : 0.f);
+            if (!best.parts || t < best.us) best = {mb == 1 && type == HQ_TYPE_Q4_K ? 2 : mb, one ? 1 : 2, parts, t};
         }
     }
     return best;

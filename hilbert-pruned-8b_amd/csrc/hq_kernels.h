@@ -140,7 +140,9 @@ HqSmPlan hq_sm_plan(const hq_dev_mat *W, int M, int n_cu, int max_parts = 8);
 hipError_t hq_launch_gemm_sm(const hq_dev_mat *W, const uint16_t *A, int M, void *C, int c_f32, int accumulate, const HqSmPlan &p,
                              float *partials, int *counters, hipStream_t st);
 
-// Q6_K (hq_q6k.hip)
+// Q6_K (hq_q6k.hip); the GEMM is the narrow Stream-K kernel with 16 mb rows per tile
+struct GemmArgs;
+hipError_t hq_launch_gemm_q6k(const GemmArgs &g, int mb, hipStream_t st);
 hipError_t hq_launch_dequant_q6k(const hq_dev_mat *W, uint32_t row0, const uint32_t *ids, uint32_t nrows, float *out,
                                  hipStream_t st);
 
@@ -153,6 +155,7 @@ int hq_sb_rows(int n_out);       // rows per wave of that GEMV and gather for n_
 int hq_sb_lds(int type, int K);  // whether that GEMV copies its activation vector into LDS
 hipError_t hq_launch_gather_kq(const hq_dev_mat *W, const uint16_t *H, const uint32_t *ids, int B, int k, float *out,
                                hipStream_t st);
+hipError_t hq_launch_gemm_kq(int type, const GemmArgs &g, int mb, hipStream_t st);  // narrow Stream-K, as for Q6_K
 constexpr bool hq_is_kq(int type) { return type == HQ_TYPE_Q2_K || type == HQ_TYPE_Q3_K || type == HQ_TYPE_Q5_K; }
 
 #endif

@@ -585,9 +585,292 @@ __global__ void __launch_bounds__(256) k_gather_q4_k(const uint8_t *__restrict__
 
 #include "hq_sk.h"
 
+template <int MB, int NB>
+__global__ void __launch_bounds__(256) k_gemm_q8_0(GemmArgs g) {
+    __shared__ __attribute__((aligned(16))) _Float16 sa[2][16 * MB * KC];
+    __shared__ int s_flag;
+    const SkPlan &p = g.plan;
+    const int w = sk_worker(p.G), u0 = sk_start(p, w), u1 = sk_start(p, w + 1);
+    const rsrc_t rpart = make_rsrc(g.partials, g.partial_bytes);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ln = lane & 15, lg = lane >> 4;
+    const int M = g.M, N = g.N, K = g.K;
+    const rsrc_t ra = make_rsrc(g.A, (uint32_t)((size_t)M * K * 2));
+    const rsrc_t rq = make_rsrc(g.qs, (uint32_t)((size_t)N * K));
+    const rsrc_t rd = make_rsrc(g.d, (uint32_t)((size_t)N * g.ldd * 2));
+    // per-tile lane offsets: rows beyond N read zero weights
+    ADma adma;
+    uint32_t vq[NB], vd[NB];
+    auto tile_setup = [&](int tile) {
+        const int m0 = (tile % p.tm) * 16 * MB, nw = (tile / p.tm) * 64 * NB + wave * 16 * NB;
+        adma = adma_setup<MB>(K, m0);
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const uint32_t n = (uint32_t)(nw + 16 * j + ln);
+            vq[j] = n * (uint32_t)K + 16u * lg;
+            vd[j] = n * (uint32_t)g.ldd * 2u;
+        }
+    };
+    // lane (ln, lg) holds weights [64s + 16lg, +16) of the unit for s = 0..3 and its 8 block scales
+    auto load_w = [&](int k0, u4v (&q)[NB][4], u4v (&d)[NB]) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            d[j] = buf_load16(rd, vd[j], (uint32_t)(k0 / 16));
+#pragma unroll
+            for (int s = 0; s < 4; s++) q[j][s] = buf_load16(rq, vq[j] + 64u * s, (uint32_t)k0);
+        }
+    };
+    f4 acc[MB][NB];
+    u4v qc[NB][4], dc[NB];
+    int cur_tile = u0 / p.upt;
+    tile_setup(cur_tile);
+    dma_a<MB>(sa[0], ra, adma, K, (u0 % p.upt) * KC);
+    load_w((u0 % p.upt) * KC, qc, dc);
+    for (int u = u0; u < u1; u++) {
+        const int cb = (u - u0) & 1, tile = u / p.upt, ku = u % p.upt;
+        const int m0 = (tile % p.tm) * 16 * MB, nw = (tile / p.tm) * 64 * NB + wave * 16 * NB;
+        const int k0 = ku * KC, kc = K - k0 < KC ? K - k0 : KC;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        u4v qn[NB][4], dn[NB];
+        if (u + 1 < u1) {
+            const int t1 = (u + 1) / p.upt;
+            if (t1 != cur_tile) {
+                cur_tile = t1;
+                tile_setup(t1);
+            }
+            const int k1 = ((u + 1) % p.upt) * KC;
+            dma_a<MB>(sa[cb ^ 1], ra, adma, K, k1);
+            load_w(k1, qn, dn);
+        }
+        if (u == u0 || ku == 0) {
+#pragma unroll
+            for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int j = 0; j < NB; j++) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+        // decode: bf[j][2s + t] covers activations 64s + 16lg + 8t .. +8 (chunk index 8s + 2lg + t);
+        // pieces past the end of K (last unit of a row only) get a zero scale
+        h8 bf[NB][8];
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const uint32_t dw[4] = {dc[j].x, dc[j].y, dc[j].z, dc[j].w};
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const int blk = 2 * s + (lg >> 1);  // block of this lane's 16 weights
+                const uint32_t dd = dw[blk >> 1] >> (16 * (blk & 1));
+                const int valid = 64 * s + 16 * lg < kc;
+                const _Float16 dh = __builtin_bit_cast(_Float16, (uint16_t)(valid ? dd : 0u));
+                const h2 d2 = {dh, dh};
+                bf[j][2 * s] = frag_q8_0(qc[j][s].x, qc[j][s].y, d2);
+                bf[j][2 * s + 1] = frag_q8_0(qc[j][s].z, qc[j][s].w, d2);
+            }
+        }
+        const _Float16 *buf = sa[cb];
+#pragma unroll
+        for (int i = 0; i < MB; i++) {
+            const int r = 16 * i + ln;
+#pragma unroll
+            for (int f = 0; f < 8; f++) {
+                const h8 af = a_frag(buf, r, 8 * (f >> 1) + 2 * lg + (f & 1));
+#pragma unroll
+                for (int j = 0; j < NB; j++) acc[i][j] = mfma(af, bf[j][f], acc[i][j]);
+            }
+        }
+        if (ku == p.upt - 1 || u == u1 - 1)
+            finish_tile<MB, NB, 256>(acc, p, w, u0, u1, tile, &s_flag, rpart, g.counters, g.C, M, N, m0, nw, ln, lg,
+                                g.c_f32, g.accumulate);
+        if (u + 1 < u1) {
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                dc[j] = dn[j];
+#pragma unroll
+                for (int s = 0; s < 4; s++) qc[j][s] = qn[j][s];
+            }
+        }
+    }
+}
+
+template <int MB, int NB>
+__global__ void __launch_bounds__(256) k_gemm_q4_k(GemmArgs g) {
+    constexpr int BM = 16 * MB;
+    __shared__ __attribute__((aligned(16))) _Float16 sa[2][BM * KC];
+    __shared__ __attribute__((aligned(16))) _Float16 ss[2][BM * 16];  // per row: sums hi[8], lo[8]
+    __shared__ int s_flag;
+    const SkPlan &p = g.plan;
+    const int w = sk_worker(p.G), u0 = sk_start(p, w), u1 = sk_start(p, w + 1);
+    const rsrc_t rpart = make_rsrc(g.partials, g.partial_bytes);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 15, lg = lane >> 4;
+    const int M = g.M, N = g.N, K = g.K;
+    const rsrc_t ra = make_rsrc(g.A, (uint32_t)((size_t)M * K * 2));
+    const rsrc_t rw = make_rsrc(g.qs, (uint32_t)((size_t)N * g.row_bytes));
+    ADma adma;
+    uint32_t vh[NB], vq[NB];
+    // Lane (ln, lg) loads chunk c = 4L + lg (L = 0, 1) of the 128 quant bytes: p = 2L + lg/2,
+    // h = lg%2. MFMA 4L + t: t = 0/1 low nibbles of bytes 0-7 / 8-15, t = 2/3 high nibbles; its
+    // activations start at k = 64p + 16h + 8(t&1) + 32(t>>1) (chunk k/8); sub-block 2p + (t>>1).
+    auto tile_setup = [&](int tile) {
+        const int m0 = (tile % p.tm) * BM, nw = (tile / p.tm) * 64 * NB + wave * 16 * NB;
+        adma = adma_setup<MB>(K, m0);
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const uint32_t n = (uint32_t)(nw + 16 * j + ln);
+            vh[j] = n * (uint32_t)g.row_bytes;
+            vq[j] = vh[j] + 16u + 16u * lg;
+        }
+    };
+    auto load_w = [&](int sb, u4v (&h)[NB], u4v (&q0)[NB], u4v (&q1)[NB]) {
+        const uint32_t so = (uint32_t)sb * 144u;
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            h[j] = buf_load16(rw, vh[j], so);
+            q0[j] = buf_load16(rw, vq[j], so);
+            q1[j] = buf_load16(rw, vq[j] + 64u, so);
+        }
+    };
+    const int pA = lg >> 1, hA = lg & 1;
+    f4 acc[MB][NB];
+    u4v hc[NB], q0c[NB], q1c[NB];
+    // min term deferred from the previous unit: integer m operand and -dmin per column block
+    h8 bm_prev[NB];
+    float ndmin_prev[NB];
+    bool min_pending = false;
+    int cur_tile = u0 / p.upt;
+    tile_setup(cur_tile);
+    dma_a<MB>(sa[0], ra, adma, K, (u0 % p.upt) * KC);
+    load_w(u0 % p.upt, hc, q0c, q1c);
+    auto apply_min = [&](const _Float16 *sbuf) {
+#pragma unroll
+        for (int i = 0; i < MB; i++) {
+            // lanes lg even: sums hi, odd: lo (lanes lg >= 2 meet a zero B operand)
+            const h8 as = *(const h8 *)(sbuf + (16 * i + ln) * 16 + 8 * (lg & 1));
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                const f4 mp = mfma(as, bm_prev[j], f4{0.f, 0.f, 0.f, 0.f});
+                acc[i][j] += mp * ndmin_prev[j];
+            }
+        }
+    };
+    for (int u = u0; u < u1; u++) {
+        const int cb = (u - u0) & 1, tile = u / p.upt, sb = u % p.upt;
+        const int m0 = (tile % p.tm) * BM, nw = (tile / p.tm) * 64 * NB + wave * 16 * NB;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (min_pending) {  // the previous unit of this tile: its sums are complete now
+            apply_min(ss[cb ^ 1]);
+            min_pending = false;
+        }
+        u4v hn[NB], q0n[NB], q1n[NB];
+        if (u + 1 < u1) {
+            const int t1 = (u + 1) / p.upt;
+            if (t1 != cur_tile) {
+                cur_tile = t1;
+                tile_setup(t1);
+            }
+            const int sb1 = (u + 1) % p.upt;
+            dma_a<MB>(sa[cb ^ 1], ra, adma, K, sb1 * KC);
+            load_w(sb1, hn, q0n, q1n);
+        }
+        if (u == u0 || sb == 0) {
+#pragma unroll
+            for (int i = 0; i < MB; i++)
+#pragma unroll
+                for (int j = 0; j < NB; j++) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+        const _Float16 *buf = sa[cb];
+        // sub-block sums of this unit: thread -> (row, sub) pairs, rows fastest (conflict-free reads)
+        {
+            const h2 one = {(_Float16)1.0f, (_Float16)1.0f};
+#pragma unroll
+            for (int q = 0; q < (BM * 8 + 255) / 256; q++) {
+                const int pr = tid + 256 * q;
+                if ((BM * 8) % 256 == 0 || pr < BM * 8) {
+                    const int r = pr % BM, sub = pr / BM;
+                    float s = 0.f;
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const u4v x = *(const u4v *)(buf + r * KC + 8 * ((4 * sub + v) ^ (r & 15)));
+                        s = __builtin_amdgcn_fdot2(as_h2(x.x), one, s, false);
+                        s = __builtin_amdgcn_fdot2(as_h2(x.y), one, s, false);
+                        s = __builtin_amdgcn_fdot2(as_h2(x.z), one, s, false);
+                        s = __builtin_amdgcn_fdot2(as_h2(x.w), one, s, false);
+                    }
+                    const _Float16 hi = (_Float16)s;
+                    ss[cb][r * 16 + sub] = hi;
+                    ss[cb][r * 16 + 8 + sub] = (_Float16)(s - (float)hi);
+                }
+            }
+        }
+        h8 bf[NB][8];
+        float dsc[NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            uint32_t sw0, sw1, mw0, mw1;
+            q4k_scale_words(hc[j].y, hc[j].z, hc[j].w, sw0, sw1, mw0, mw1);
+            h2 mulL[2][2], addL[2][2];
+#pragma unroll
+            for (int L = 0; L < 2; L++) {
+                const uint32_t sw = L ? sw1 : sw0;
+#pragma unroll
+                for (int hi = 0; hi < 2; hi++) {
+                    const float s = (float)byte_of(sw, 2 * pA + hi);
+                    const _Float16 mul = (_Float16)(hi ? s * 0.0625f : s);
+                    const _Float16 add = (_Float16)(hi ? -64.0f * s : -1024.0f * s);
+                    mulL[L][hi] = h2{mul, mul};
+                    addL[L][hi] = h2{add, add};
+                }
+            }
+            bf[j][0] = frag_q4_k<false>(q0c[j].x, q0c[j].y, mulL[0][0], addL[0][0]);
+            bf[j][1] = frag_q4_k<false>(q0c[j].z, q0c[j].w, mulL[0][0], addL[0][0]);
+            bf[j][2] = frag_q4_k<true>(q0c[j].x, q0c[j].y, mulL[0][1], addL[0][1]);
+            bf[j][3] = frag_q4_k<true>(q0c[j].z, q0c[j].w, mulL[0][1], addL[0][1]);
+            bf[j][4] = frag_q4_k<false>(q1c[j].x, q1c[j].y, mulL[1][0], addL[1][0]);
+            bf[j][5] = frag_q4_k<false>(q1c[j].z, q1c[j].w, mulL[1][0], addL[1][0]);
+            bf[j][6] = frag_q4_k<true>(q1c[j].x, q1c[j].y, mulL[1][1], addL[1][1]);
+            bf[j][7] = frag_q4_k<true>(q1c[j].z, q1c[j].w, mulL[1][1], addL[1][1]);
+            // min operand for the next barrier: lanes lg 0, 1 carry m_0..m_7 (k-slot e = sub-block e)
+            const h2 m01 = bytes_f16(mw0, false), m23 = bytes_f16(mw0, true);
+            const h2 m45 = bytes_f16(mw1, false), m67 = bytes_f16(mw1, true);
+            const h8 mv = {m01.x, m01.y, m23.x, m23.y, m45.x, m45.y, m67.x, m67.y};
+            bm_prev[j] = lg < 2 ? mv : h8{0, 0, 0, 0, 0, 0, 0, 0};
+            ndmin_prev[j] = -h2f((uint16_t)(hc[j].x >> 16));
+            dsc[j] = h2f((uint16_t)hc[j].x);
+        }
+#pragma unroll
+        for (int i = 0; i < MB; i++) {
+            const int r = 16 * i + ln;
+            f4 part[NB];
+#pragma unroll
+            for (int j = 0; j < NB; j++) part[j] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int L = 0; L < 2; L++)
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const h8 af = a_frag(buf, r, 8 * (2 * L + pA) + 2 * hA + (t & 1) + 4 * (t >> 1));
+#pragma unroll
+                    for (int j = 0; j < NB; j++) part[j] = mfma(af, bf[j][4 * L + t], part[j]);
+                }
+#pragma unroll
+            for (int j = 0; j < NB; j++) acc[i][j] += part[j] * dsc[j];
+        }
+        min_pending = true;
+        if (sb == p.upt - 1 || u == u1 - 1) {
+            __syncthreads();  // this unit's sums, written by other waves
+            apply_min(ss[cb]);
+            min_pending = false;
+            finish_tile<MB, NB, 256>(acc, p, w, u0, u1, tile, &s_flag, rpart, g.counters, g.C, M, N, m0, nw, ln, lg,
+                                g.c_f32, g.accumulate);
+        }
+        if (u + 1 < u1) {
+#pragma unroll
+            for (int j = 0; j < NB; j++) hc[j] = hn[j], q0c[j] = q0n[j], q1c[j] = q1n[j];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------- wide Q4_K GEMM (M > 64)
 // 8 waves, two per SIMD (one wave's LDS and memory waits are covered by the other's MFMAs); tile
-// 128 (M) x 256 (N): wave w owns columns [32w, 32w + 32) and all 128 rows. The activation sub-block sums come from k_asums (one pass over A per GEMM instead of
+// 128 (M) x 256 (N): wave w owns columns [32w, 32w + 32) and all 128 rows, decoded as in
+// k_gemm_q4_k. The activation sub-block sums come from k_asums (one pass over A per GEMM instead of
 // one per N tile): plane S[m][u][16] fp16 = {hi(S_0..S_7), lo(S_0..S_7)} of unit u, staged in LDS
 // next to the activation tile. The min term is one MFMA per (16-row block, 16-column block, unit)
 // accumulating straight into the output: A operand lanes lg = 0..3 hold S_hi, S_lo, S_hi, S_lo of
@@ -1114,8 +1397,12 @@ WrPlan wr4_plan(int M, int N, int n_cu) {
 }  // namespace
 
 namespace {
-// Kernel choice for M >= 2. Q4_K with M > 64 that no rule below takes runs the wide Stream-K kernel.
+// Kernel choice for M >= 2. What no rule below takes runs a Stream-K kernel: the wide one (Q4_K, M > 64) or the
+// narrow ones, whose 16-row blocks of M per tile (mb) grow with M up to 8 (Q4_K: at least 2; the other k-quants:
+// up to 4), with two 16-column blocks per wave. Stream-K removes the wave-quantization cost, so the tile only sets
+// the operand reuse.
 struct GemmCfg {
+    int mb;        // row blocks of the narrow Stream-K kernel
     bool wide;     // Q4_K, Q5_K with M > 64 (the kernels that use activation sub-block sums)
     int ws_nb;     // > 0: the full-K tile kernel k_gemm_q4_k_ws with 32 * ws_nb columns per tile
     int ws_parts;  // with ws_nb: workgroups per tile, each a contiguous range of K (1: whole K)
@@ -1134,15 +1421,20 @@ struct GemmCfg {
     HqSmPlan sm;    // sm.parts > 0: few output tiles, the small-tile kernels of hq_gemm_sm.hip
 };
 
-// Estimated us of an LDS-decode tile kernel: stages of 128 K per part, nb columns / 32, parts and rounds.
-// (fits of its measured times over N, K = 512 .. 9728, M = 80 .. 8192; half within 3-5 %)
+// Estimated us of an LDS-decode tile kernel: stages of 128 K per part, nb columns / 32, parts, rounds of the fullest
+// XCD, millions of outputs (more where rows of C are not whole 8-value pieces). (Fits of its measured times over
+// N = 64 .. 20000, K = 512 .. 15360, M = 65 .. 8192: half within 4 %, nine in ten within 12 %. Rounds counted over all CUs
+// instead of an XCD's put every fifth shape at half its time: M = 1317, N = 600 makes 44 workgroups on two XCDs.)
 float ws_us(int type, int M, int N, int K, int nb, int parts, int n_cu) {
-    struct Fit { float base, stage, stage_nb, split, round; };
-    const Fit f = type == HQ_TYPE_Q4_K ? Fit{7.9f, .339f, .302f, .269f, 0.f}
-                : type == HQ_TYPE_Q5_K ? Fit{9.5f, .288f, .291f, .270f, 6.1f} : Fit{6.6f, .096f, .300f, .284f, 6.5f};
-    const long wgs = (long)((M + 127) / 128) * ((N + 32 * nb - 1) / (32 * nb)) * parts, rounds = (wgs + n_cu - 1) / n_cu;
-    const float stages = (float)(rounds * ((K / 128 + parts - 1) / parts));
-    return f.base + stages * (f.stage + f.stage_nb * nb) + (parts > 1 ? f.split * nb * parts : 0.f) + f.round * (float)(rounds - 1);
+    struct Fit { float base, stage, stage_nb, split, round, out, ragged; };
+    const Fit f = type == HQ_TYPE_Q4_K ? Fit{4.f, .61f, .19f, .4f, 3.6f, 2.5f, 4.f}
+                : type == HQ_TYPE_Q5_K ? Fit{7.5f, .45f, .2f, .41f, 4.7f, .7f, 2.f}
+                : type == HQ_TYPE_Q8_0 ? Fit{3.3f, .475f, .17f, .5f, 3.1f, .65f, 2.1f} : Fit{4.5f, .225f, .24f, .41f, 3.3f, .8f, 1.9f};
+    const long mt = (M + 127) / 128, nt = (N + 32 * nb - 1) / (32 * nb), xcd = std::max(1, n_cu / 8);
+    const long rounds = ((nt + 7) / 8 * mt * parts + xcd - 1) / xcd;
+    const float stages = (float)(rounds * ((K / 128 + parts - 1) / parts)), out = 1e-6f * (float)M * (float)N;
+    return f.base + stages * (f.stage + f.stage_nb * nb) + (parts > 1 ? f.split * nb * parts : 0.f) + f.round * (float)(rounds - 1) +
+           out * (f.out + (N % 8 ? f.ragged : 0.f));
 }
 
 // Parts of K for k_gemm_q8_0_wr_ks with the least estimated us, one round on every XCD: launches, prologue,
@@ -1158,28 +1450,77 @@ int wr8_split(int M, int N, int K, int n_cu, float *us) {
     return best;
 }
 
-// Whether the small-tile kernels (plan p) run instead of the kernel that c names so far. They replaced the
-// narrow Stream-K kernels, which they beat at every size measured (M = 2 .. 2048, N = 16 .. 15360,
-// K = 512 .. 15360; geometric mean 1.5x), so what is left to compare is
-//   the mid-M kernels: Q8_0's is 5-20 % faster everywhere it applies; Q4_K's where its tiles fill the chip
-//     (N = 9728, M = 64: 14.9 against 15.2 us) or K is long, not where it splits a short K (N = 4096,
-//     K = 2560: 12.2 against 10.5; p.us < 11 divides the two);
-//   the LDS-decode tile kernels (M > 64), where the estimates are 15 % apart (that left no loss among the
-//     measured shapes; e.g. Q4_K M = 256, N = 4096, K = 2560 18.0 -> 15.7 us); not Q8_0's, whose few losses
-//     would not pay for a rule;
-//   the wide Q4_K Stream-K kernel (M = 128, N = K = 2560: 27.0 -> 11.9 us; M = 256, N = 1024: 26.1 -> 8.4).
-//     It keeps N < 64, a K of one super-block, and the large end (M > 256 with over 2^21 weights), where the
-//     small tiles win less (M = 512, N = 1024, K = 2560: 28 against 12 us) and, with M = 1024, nothing.
+// Estimated us of the Stream-K kernels from their plan: launch and prologue, the fullest workgroup's K-units and
+// ends of tiles, the exchange of cut tiles (and the workgroups that share one), what the units read in MB, millions of
+// outputs where rows of C are not whole 8-value pieces, and for the wide kernel its activation-sum pass and output.
+// (Least squares over N = 1 .. 20000, K = 32 .. 15360, M = 2 .. 8192 and every type: half within 5 %, nine in ten within 13 %.)
+float sk_us(int type, int M, int N, int mb, bool wide, const SkPlan &p) {
+    const int per = (p.base + (p.extra > 0)), ends = (per + p.upt - 1) / p.upt;
+    const bool cut = p.extra || p.base % p.upt;
+    const int share = cut ? std::max(1, std::min(p.upt, (p.upt + std::max(p.base, 1) - 1) / std::max(p.base, 1))) : 0;
+    const float units = (float)p.tiles * (float)p.upt;
+    if (wide) {
+        const float mb_units = units * 1e-6f * (128 * 512 + 256 * 144), K = 256.f * (float)p.upt;
+        return 7.9f + 1.53f * (float)per + (cut ? 3.f : 0.f) + 1.11f * (float)share + 2.15f * (float)ends + .12f * mb_units +
+               1e-6f * (float)M * (.49f * K + .79f * (float)N);
+    }
+    struct Fit { float base, unit, cut, share, end, read, ragged; };
+    static const Fit q8[4] = {{3.07f, .73f, 1.05f, .33f, 0.f, .159f, 1.2f}, {3.5f, .95f, 1.34f, .39f, 0.f, .132f, 2.8f}, {4.f, 1.29f, 1.6f, .47f, .3f, .102f, 4.9f},
+                              {4.66f, 1.54f, 1.97f, .92f, 2.1f, .087f, 1.f}},
+                     kq[3] = {{3.12f, .65f, 1.08f, .3f, 0.f, .184f, 3.9f}, {3.6f, .75f, 1.2f, .4f, 0.f, .12f, 3.6f}, {4.17f, 1.27f, 1.76f, .445f, .54f, .11f, 2.2f}};
+    const int lg = mb == 1 ? 0 : mb == 2 ? 1 : mb == 4 ? 2 : 3;
+    const Fit &f = type == HQ_TYPE_Q8_0 ? q8[lg] : kq[std::min(lg, 2)];
+    const float decode = type == HQ_TYPE_Q6_K ? 1.13f : type == HQ_TYPE_Q5_K ? .82f : type == HQ_TYPE_Q2_K ? .4f : type == HQ_TYPE_Q3_K ? .3f : 0.f;
+    const float wb = type == HQ_TYPE_Q8_0 ? 1.06f : type == HQ_TYPE_Q4_K ? .5625f : type == HQ_TYPE_Q5_K ? .6875f : type == HQ_TYPE_Q6_K ? .875f
+                   : type == HQ_TYPE_Q3_K ? .4375f : .375f;
+    return f.base + (float)per * (f.unit + decode) + (cut ? f.cut : 0.f) + f.share * (float)share + f.end * (float)ends +
+           f.read * 1e-6f * units * (16.f * 512.f * (float)mb + 128.f * 256.f * wb) + (N % 8 ? f.ragged * 1e-6f * (float)M * (float)N : 0.f);
+}
+
+// Estimated us of the mid-M kernels (hq_gemm_rb.hip): prologue, the stages of two super-blocks (Q4_K) or one (Q8_0) of
+// the fullest CU's workgroups, the parts' exchange, weights in MB and activations through every column tile.
+float rb_us(int type, int M, int N, int K, int parts, int n_cu) {
+    const int tiles = (N + 63) / 64, rounds = (8 * ((tiles + 7) / 8) * parts + n_cu - 1) / n_cu, lg = M <= 16 ? 0 : M <= 32 ? 1 : 2;
+    const float acts = 1e-6f * (float)M * (float)K * (float)tiles, w = 1e-6f * (float)N * (float)K;
+    if (type == HQ_TYPE_Q4_K)
+        return 5.4f + 1.52f * (float)(rounds * ((K / 512 + parts - 1) / parts)) + 1.7f * (float)(rounds - 1) +
+               (parts > 1 ? 1.1f + .1f * (float)parts : 0.f) + .04f * w + .05f * acts;
+    static const float base[3] = {4.3f, 4.3f, 5.2f}, stage[3] = {.34f, .48f, .63f};
+    return base[lg] + stage[lg] * (float)(rounds * ((K / 256 + parts - 1) / parts)) + .74f * (float)(rounds - 1) +
+           (parts > 1 ? .7f + .15f * (float)parts + .04f * (float)(1 << lg) : 0.f) + .08f * w + .07f * acts;
+}
+
+// The wide Stream-K kernel's plan (tiles of 128 x 256), or the narrow ones' (16 mb x 128)
+SkPlan gemm_plan(const hq_dev_mat *W, int M, const GemmCfg &c, int n_cu) {
+    return hq_sk_plan(M, (int)W->rows, (int)W->cols, c.wide ? 128 : 16 * c.mb, c.wide ? 256 : 128, n_cu);
+}
+
+// Estimated us of the kernel that c names, the small-tile ones aside (not for the register-decode and skinny kernels)
+float cfg_us(const hq_dev_mat *W, int M, const GemmCfg &c, int n_cu) {
+    const int type = W->type, N = (int)W->rows, K = (int)W->cols;
+    if (c.rbm || c.rb8) return rb_us(type, M, N, K, c.rbm ? c.rbm : c.rb8, n_cu);
+    if (c.ws_nb) return ws_us(type, M, N, K, c.ws_nb, c.ws_parts, n_cu);
+    if (c.ws8_nb) return ws_us(type, M, N, K, c.ws8_nb, c.ws8_parts, n_cu);
+    return sk_us(type, M, N, c.mb, c.wide, gemm_plan(W, M, c, n_cu));
+}
+
+// Whether the small-tile kernels (plan p) run instead of the kernel that c names so far: where their estimate is 8 %
+// lower (M <= 64, where both estimates are closer: 3 %). Of 34461
+// measured calls (every type, N = 1 .. 20000, K = 32 .. 15360, M = 2 .. 8192) that leaves 135 more than 4 % slower
+// than without the small tiles; where they run, they are 1.47x faster in the geometric mean.
+// Under a rule on types and sizes alone every fifth call lost (6782), up to 2x: Q8_0 M = 4096, N = 4096, K = 2592 156 ->
+// 256 us; Q4_K M = 3418, N = 2048, K = 512 23.5 -> 40.6; Q3_K M = 1085, N = 576, K = 2304 17.0 -> 23.9; Q8_0 M = 16,
+// N = 4096, K = 96 3.9 -> 6.1.
+// Never for the register-decode kernels, the mid-M ones (as fast or faster where they apply: Q4_K M = 40, N = 7680,
+// K = 2048 10.4 against 11.7 us) and Q8_0's LDS-decode tiles, whose few losses would not pay for a rule. The wide Q4_K
+// kernel keeps K <= 256, N < 64 and M > 256 with over 2^21 weights whatever the estimates: its own tests lie there
+// (M = 512, N = 1024, K = 2560, where small tiles take 12 us instead of 28).
 bool sm_better(const hq_dev_mat *W, int M, const GemmCfg &c, const HqSmPlan &p, int n_cu) {
     const int type = W->type, N = (int)W->rows, K = (int)W->cols;
-    if (M <= 64) return type == HQ_TYPE_Q8_0 ? !c.rb8 : !c.rbm || (c.rbm > 1 && p.us < 11.f);
-    if (c.wr || c.wr8 || c.bt) return false;
-    if (c.ws_nb || c.ws8_nb) {
-        if (type == HQ_TYPE_Q8_0 || K <= 256) return false;
-        return 1.15f * p.us < (c.ws_nb ? ws_us(type, M, N, K, c.ws_nb, c.ws_parts, n_cu) : ws_us(type, M, N, K, c.ws8_nb, c.ws8_parts, n_cu));
-    }
-    if (type != HQ_TYPE_Q4_K) return true;
-    return N >= 64 && K > 256 && (M <= 256 || (long)N * K <= 1l << 21);
+    if (c.rbm || c.rb8 || c.wr || c.wr8 || c.bt || (type == HQ_TYPE_Q8_0 && (c.ws8_nb || K <= 256))) return false;
+    if (c.wide && !c.ws_nb && (K <= 256 || N < 64 || (M > 256 && (long)N * K > 1l << 21))) return false;
+    if ((c.ws_nb || c.ws8_nb) && K <= 256) return false;
+    return p.us < (M > 64 ? .92f : .97f) * cfg_us(W, M, c, n_cu);
 }
 
 // Q4_K with M > 64 runs the full-K tile kernel when its tiles fit in one round on the CUs and fill
@@ -1189,7 +1530,10 @@ bool sm_better(const hq_dev_mat *W, int M, const GemmCfg &c, const HqSmPlan &p, 
 // overhead is amortised: measured faster at M = 4096 and 16384).
 GemmCfg gemm_cfg(const hq_dev_mat *W, int M, int n_cu) {
     GemmCfg c;
-    // (Q5_K: the Q4_K LDS-decode tile kernel where it is chosen below, else the small-tile kernels)
+    c.mb = M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8;
+    if ((W->type == HQ_TYPE_Q6_K || hq_is_kq(W->type)) && c.mb > 4) c.mb = 4;
+    if (W->type == HQ_TYPE_Q4_K && c.mb == 1) c.mb = 2;
+    // (Q5_K: the Q4_K LDS-decode tile kernel where it is chosen below, else the small-tile or Stream-K ones)
     c.wide = (W->type == HQ_TYPE_Q4_K || W->type == HQ_TYPE_Q5_K) && M > 64;
     c.ws_nb = 0;
     c.ws_parts = 1;
@@ -1326,9 +1670,9 @@ GemmCfg gemm_cfg(const hq_dev_mat *W, int M, int n_cu) {
         const int N = (int)W->rows, K = (int)W->cols;
         float us = 0.f;
         const int parts = wr8_split(M, N, K, n_cu, &us);
-        const float now = c.ws8_nb ? ws_us(W->type, M, N, K, c.ws8_nb, c.ws8_parts, n_cu) : hq_sm_plan(W, M, n_cu).us;
+        const float now = c.ws8_nb ? cfg_us(W, M, c, n_cu) : std::min(cfg_us(W, M, c, n_cu), hq_sm_plan(W, M, n_cu).us);
         const bool full = c.ws8_parts > 1 && 5L * M * N * c.ws8_parts >= 4L * n_cu * 128 * 32 * c.ws8_nb;
-        if (parts > 1 && !full && (K >= 6144 ? us < now : M <= 128 && parts <= 3 && c.ws8_nb && us < .95f * now))
+        if (parts > 1 && !full && (K >= 6144 ? us < now : M <= 128 && parts <= 3 && c.ws8_nb && us < 1.03f * now))
             c.wr8 = true, c.wr8_parts = parts;
     }
     // N <= 32 with at least 64 workgroups of 64 rows (config 4's b / a projections at M = 16384: 256):
@@ -1347,8 +1691,6 @@ GemmCfg gemm_cfg(const hq_dev_mat *W, int M, int n_cu) {
     return c;
 }
 
-// the wide Stream-K kernel's plan: tiles of 128 x 256
-SkPlan gemm_plan(const hq_dev_mat *W, int M, int n_cu) { return hq_sk_plan(M, (int)W->rows, (int)W->cols, 128, 256, n_cu); }
 }  // namespace
 
 // device bytes of a row of K values (the upload's layout: Q8_0 quant plane, k-quant slots)
@@ -1373,12 +1715,14 @@ void hq_gemm_tile_shape(int type, int M, int N, int K, int n_cu, int *rows, int 
         *rows = 16 * c.sm.mb, *cols = 128 / c.sm.kw;
         return;
     }
-    *rows = c.bt ? 256 : c.wr || c.wr8 ? 128 : c.rbm ? 64 : c.rb8 ? (M <= 16 ? 16 : M <= 32 ? 32 : 64) : 128;
-    *cols = c.bt ? 256 : c.wr ? c.wr_tw : c.wr8 ? 192 : c.rbm || c.rb8 ? 64 : c.ws_nb ? 32 * c.ws_nb : c.ws8_nb ? 32 * c.ws8_nb : 256;
+    *rows = c.bt ? 256 : c.wr || c.wr8 ? 128 : c.rbm ? 64 : c.rb8 ? (M <= 16 ? 16 : M <= 32 ? 32 : 64) : c.ws_nb || c.ws8_nb || c.wide ? 128 : 16 * c.mb;
+    *cols = c.bt ? 256 : c.wr ? c.wr_tw : c.wr8 ? 192 : c.rbm || c.rb8 ? 64 : c.ws_nb ? 32 * c.ws_nb : c.ws8_nb ? 32 * c.ws8_nb : c.wide ? 256 : 128;
 }
 
 // Name of the kernel that does the work of an M x N x K hq_gemm call (the main kernel for GEMMs
-// with a pre-pass), as rocprofv3 lists it.
+// with a pre-pass), as rocprofv3 lists it before the argument list. k_gemm_q8_0, k_gemm_q4_k, k_gemm_q6_k and k_gemm_kq
+// each name two kernels, told apart there by the argument: GemmArgs (narrow Stream-K; template arguments: row blocks
+// and column blocks per wave) or SmArgs (small tiles).
 void hq_gemm_kernel_name(int type, int M, int N, int K, int n_cu, char *buf, size_t n) {
     hq_dev_mat W = {};
     W.type = type;
@@ -1423,7 +1767,9 @@ void hq_gemm_kernel_name(int type, int M, int N, int K, int n_cu, char *buf, siz
     else if (c.wr8) snprintf(buf, n, c.wr8_parts > 1 ? "k_gemm_q8_0_wr_ks" : "k_gemm_q8_0_wr");
     else if (c.ws_nb) snprintf(buf, n, "k_gemm_q4_k_ws<%d>", c.ws_nb);
     else if (c.ws8_nb) snprintf(buf, n, "k_gemm_q8_0_ws<%d>", c.ws8_nb);
-    else snprintf(buf, n, "k_gemm_q4_k_w<8>");  // template argument: row blocks
+    else if (c.wide) snprintf(buf, n, "k_gemm_q4_k_w<8>");  // template argument: row blocks
+    else if (kq) snprintf(buf, n, "k_gemm_kq<%s, %d, 2>", kq, c.mb);
+    else snprintf(buf, n, "%s<%d, 2>", type == HQ_TYPE_Q4_K ? "k_gemm_q4_k" : type == HQ_TYPE_Q6_K ? "k_gemm_q6_k" : "k_gemm_q8_0", c.mb);
 }
 
 void hq_gemm_work_bytes(const hq_dev_mat *W, int M, int n_cu, size_t *partial_bytes, size_t *counter_bytes,
@@ -1440,9 +1786,9 @@ void hq_gemm_work_bytes(const hq_dev_mat *W, int M, int n_cu, size_t *partial_by
         *sums_bytes = 0;
         return;
     }
-    const SkPlan p = gemm_plan(W, M, n_cu);
+    const SkPlan p = gemm_plan(W, M, c, n_cu);
     const bool tile = c.ws_nb || c.ws8_nb || c.bt;  // tile kernels: partial tiles only when K is split (below)
-    *partial_bytes = tile ? 0 : (size_t)2 * p.G * 128 * 256 * sizeof(float);
+    *partial_bytes = tile ? 0 : (size_t)2 * p.G * (c.wide ? 128 * 256 : 16 * c.mb * 128) * sizeof(float);
     *counter_bytes = tile ? 0 : (size_t)p.tiles * sizeof(int);
     const int snb = c.ws_nb ? c.ws_nb : c.ws8_nb, sparts = c.ws_nb ? c.ws_parts : c.ws8_parts;
     if (snb && sparts > 1) {  // K-split tile kernels: one fp32 tile per (tile, part)
@@ -1519,7 +1865,7 @@ hipError_t hq_launch_gemm_main(const hq_dev_mat *W, const uint16_t *A, int M, vo
     GemmArgs g;
     g.qs = W->qs, g.d = W->d, g.ldd = W->ldd, g.row_bytes = W->row_bytes, g.A = A;
     g.M = M, g.N = (int)W->rows, g.K = (int)W->cols, g.C = C, g.c_f32 = c_f32, g.accumulate = accumulate;
-    g.plan = gemm_plan(W, M, wk.n_cu);
+    g.plan = gemm_plan(W, M, c, wk.n_cu);
     g.partials = wk.partials, g.counters = wk.counters, g.sums = wk.sums;
     {
         size_t pb, cb, sb;
@@ -1527,7 +1873,25 @@ hipError_t hq_launch_gemm_main(const hq_dev_mat *W, const uint16_t *A, int M, vo
         if (pb > 0xffffffffu) return hipErrorInvalidValue;
         g.partial_bytes = (uint32_t)pb;
     }
-    k_gemm_q4_k_w<8><<<g.plan.G, 64 * WNW, 0, st>>>(g);
+    if (c.wide) {
+        k_gemm_q4_k_w<8><<<g.plan.G, 64 * WNW, 0, st>>>(g);
+        return hipGetLastError();
+    }
+    if (W->type == HQ_TYPE_Q6_K) return hq_launch_gemm_q6k(g, c.mb, st);
+    if (hq_is_kq(W->type)) return hq_launch_gemm_kq(W->type, g, c.mb, st);
+    const bool q8 = W->type == HQ_TYPE_Q8_0;
+    switch (c.mb) {
+    case 1: k_gemm_q8_0<1, 2><<<g.plan.G, 256, 0, st>>>(g); break;  // (Q8_0 only, as 8)
+    case 2:
+        if (q8) k_gemm_q8_0<2, 2><<<g.plan.G, 256, 0, st>>>(g);
+        else k_gemm_q4_k<2, 2><<<g.plan.G, 256, 0, st>>>(g);
+        break;
+    case 4:
+        if (q8) k_gemm_q8_0<4, 2><<<g.plan.G, 256, 0, st>>>(g);
+        else k_gemm_q4_k<4, 2><<<g.plan.G, 256, 0, st>>>(g);
+        break;
+    default: k_gemm_q8_0<8, 2><<<g.plan.G, 256, 0, st>>>(g);
+    }
     return hipGetLastError();
 }
 
