@@ -505,11 +505,12 @@ int device_cus(int device, int *n_cu) {
 
 // GEMM workspace of an M-row hq_gemm on W's device and `stream`. A counter array that grows is
 // zeroed once here, synchronously; the kernels leave every counter back at zero.
-int gemm_work(const hq_mat *W, int M, void *stream, HqGemmWork *wk) {
+int gemm_work(const hq_mat *W, int M, void *stream, HqGemmWork *wk, bool swiglu = false) {
     int n_cu;
     if (device_cus(W->device, &n_cu)) return -1;
     size_t pb, cb, sb;
     hq_gemm_work_bytes(&W->m, M, n_cu, &pb, &cb, &sb);
+    if (swiglu) sb = std::max(sb, hq_swiglu_sums_bytes(&W->m, M, n_cu));
     void *part, *cnt, *sums = nullptr;
     int grew = 0;
     if (staging(W->device, stream, 5, pb, &part) || staging(W->device, stream, 6, cb, &cnt, &grew)) return -1;
@@ -642,6 +643,15 @@ extern "C" int hq_gemm_workspace_bytes(int ggml_type, int M, uint32_t N, uint32_
     return 0;
 }
 
+extern "C" int hq_internal_swiglu_small(int ggml_type, int M, uint32_t rows, uint32_t K, int n_cu) {
+    hq_dev_mat W = {};
+    W.type = ggml_type, W.rows = 2 * rows, W.cols = K;
+    const size_t nb = K / block_values(ggml_type);
+    W.row_bytes = nb * (slot_bytes(ggml_type) ? slot_bytes(ggml_type) : block_bytes(ggml_type));
+    W.ldd = ggml_type == HQ_GGML_Q8_0 ? (int)round_up(K / 32, 8) : 0;
+    return hq_swiglu_small(&W, M, n_cu);
+}
+
 extern "C" int hq_gemm_noalloc(const hq_mat *W, const uint16_t *A, int M, void *C, int c_is_f32, int accumulate,
                                void *stream) {
     if (!W || !A || !C) return fail("hq_gemm_noalloc: null argument");
@@ -708,7 +718,7 @@ extern "C" int hq_gemm_swiglu(const hq_mat *pair, const uint16_t *A, int M, uint
         if (mc == 1) {
             HIPCK(hq_launch_gemv_pair(&pair->m, Ap, Op, S(stream), &fused));
         } else {
-            if (gemm_work(pair, mc, stream, &wk)) return -1;
+            if (gemm_work(pair, mc, stream, &wk, true)) return -1;
             HIPCK(hq_launch_gemm_swiglu(&pair->m, Ap, mc, Op, wk, S(stream), &fused));
         }
         if (fused) continue;

@@ -433,7 +433,10 @@ hipError_t hq_launch_gemm_sm(const hq_dev_mat *W, const uint16_t *A, int M, void
 #define SM_LAUNCH(k) k<<<grid, SM_NT, 0, st>>>(g); break
 #define SM_CASE(mb, kw)                                                             \
     switch (W->type) {                                                              \
-    case HQ_TYPE_Q8_0: SM_LAUNCH((k_gemm_q8_0<mb, kw>));                            \
+    case HQ_TYPE_Q8_0:                                                              \
+        if constexpr (kw == 1) return hipErrorInvalidValue;                         \
+        else k_gemm_q8_0<mb, kw><<<grid, SM_NT, 0, st>>>(g);                        \
+        break;                                                                      \
     case HQ_TYPE_Q4_K: SM_LAUNCH((k_gemm_q4_k<mb == 1 ? 2 : mb, kw>));              \
     case HQ_TYPE_Q6_K: SM_LAUNCH((k_gemm_q6_k<mb, kw>));                            \
     case HQ_TYPE_Q2_K: SM_LAUNCH((k_gemm_kq<HQ_TYPE_Q2_K, mb, kw>));                \

@@ -18,6 +18,10 @@ int hq_internal_block_shape(int ggml_type, uint32_t *values, uint32_t *bytes);
 /* The accepted block types, for messages ("Q8_0 = 8, ..."). */
 const char *hq_internal_supported_types(void);
 
+/* Whether hq_gemm_swiglu on M <= 64 rows of a pair matrix of 2 * rows rows is one small-tile kernel (else hq_gemm's kernel
+ * and a pass over its product); no device is touched. */
+int hq_internal_swiglu_small(int ggml_type, int M, uint32_t rows, uint32_t K, int n_cu);
+
 /* The rows of n matrices of one type and width (Hugging Face order, one after the other) as one resident matrix. */
 int hq_internal_upload_cat(const hq_wmat_t *const *w, int n, int device, hq_mat **out);
 

@@ -70,6 +70,8 @@ hipError_t hq_launch_stream_read(const void *p, size_t bytes, uint32_t *out, uns
 // epilogue as a separate pass over an fp32 [M, 2I] product (n_out = M * I)
 hipError_t hq_launch_gemm_swiglu(const hq_dev_mat *W, const uint16_t *A, int M, uint16_t *out, const HqGemmWork &wk,
                                  hipStream_t st, int *fused);
+bool hq_swiglu_small(const hq_dev_mat *W, int M, int n_cu);  // M <= 64: whether that is a small-tile kernel
+size_t hq_swiglu_sums_bytes(const hq_dev_mat *W, int M, int n_cu);  // activation sums it needs beside hq_gemm's workspace
 hipError_t hq_launch_swiglu_pairs(const float *C, uint16_t *out, size_t n_out, hipStream_t st);
 // rows x columns of one GEMM output tile (M >= 2) on a device with n_cu CUs
 void hq_gemm_tile_shape(int type, int M, int N, int K, int n_cu, int *rows, int *cols);

@@ -1895,18 +1895,36 @@ hipError_t hq_launch_gemm_main(const hq_dev_mat *W, const uint16_t *A, int M, vo
     return hipGetLastError();
 }
 
-// gate/up pair GEMM with the SwiGLU epilogue inside the full-K tile kernels (M > 64; any number of
-// tile rounds, each tile's K in one workgroup). *fused = 0 when the shape does not suit them: the
-// caller then runs hq_launch_gemm into fp32 and hq_launch_swiglu_pairs.
+// activation sums of hq_launch_gemm_swiglu's own (Q5_K, where the LDS-decode tiles suit the shape, whatever hq_gemm runs)
+size_t hq_swiglu_sums_bytes(const hq_dev_mat *W, int M, int n_cu) {
+    return W->type == HQ_TYPE_Q5_K && M > 64 && gemm_cfg(W, M, n_cu).ws_nb ? (size_t)M * (W->cols / KC) * 32 : 0;
+}
+
+// Estimated us of the separate SwiGLU pass: its launch, and the fp32 product written and read
+float pass_us(int M, int N) { return 2.2f + 2.6e-6f * (float)M * (float)N; }
+
+// M <= 64 of a pair matrix: the small-tile kernels with the epilogue in each tile (K in one workgroup) where their estimate
+// is below that of hq_gemm's kernel (less 8 % unless that is a small-tile one too) and a pass over its fp32 product. Over 6000 calls (every type, I = 64 .. 15360): 1.37x for
+// the k-quants, nearly all of them; Q8_0 half of its calls, 1.09x, where taking every one lost up to 1.7x to the mid-M
+// kernel's K split (M = 38, I = 832, K = 3328: 11.0 -> 18.8 us). Q8_0 of one super-block: 0.79 to 1.2x, so not.
+bool hq_swiglu_small(const hq_dev_mat *W, int M, int n_cu) {
+    if (W->type == HQ_TYPE_Q8_0 && W->cols <= 256) return false;
+    const GemmCfg c = gemm_cfg(W, M, n_cu);
+    const float apart = (c.sm.parts ? c.sm.us : .92f * cfg_us(W, M, c, n_cu)) + pass_us(M, (int)W->rows);
+    return hq_sm_plan(W, M, n_cu, 1).us < apart;
+}
+
+// gate/up pair GEMM with the SwiGLU epilogue inside the small-tile kernels or the full-K tile kernels (M > 64; any number
+// of tile rounds), each tile's K in one workgroup. *fused = 0 when the shape does not suit them: the caller then runs
+// hq_launch_gemm into fp32 and hq_launch_swiglu_pairs.
 hipError_t hq_launch_gemm_swiglu(const hq_dev_mat *W, const uint16_t *A, int M, uint16_t *out, const HqGemmWork &wk,
                                  hipStream_t st, int *fused) {
     *fused = 0;
     const int N = (int)W->rows, K = (int)W->cols;
     if (N % 16) return hipSuccess;
-    // M <= 64: the small-tile kernels with the epilogue in each tile (K in one workgroup), rather than any
-    // kernel and a pass over its fp32 product
     const HqSmPlan sp = hq_sm_plan(W, M, wk.n_cu, 1);
     if (M <= 64) {
+        if (!hq_swiglu_small(W, M, wk.n_cu)) return hipSuccess;
         *fused = 1;
         return hq_launch_gemm_sm(W, A, M, out, HQ_OUT_SWIGLU, 0, sp, nullptr, nullptr, st);
     }
@@ -1937,8 +1955,9 @@ hipError_t hq_launch_gemm_swiglu(const hq_dev_mat *W, const uint16_t *A, int M, 
     }
     float eff = 0.f;
     const int nb = hq_ws_choose(M, N, wk.n_cu, &eff);
-    // against the LDS-decode tile kernels: as in sm_better
-    if (W->type != HQ_TYPE_Q8_0 && K > 256 && 1.15f * sp.us < ws_us(W->type, M, N, K, nb, 1, wk.n_cu)) {
+    // against the LDS-decode tile kernels: where the estimates are 15 % apart (1.39x over the 480 calls measured that run
+    // them; without a margin Q6_K at K = 512 .. 768 lost a tenth: M = 341, I = 1024 7.0 -> 7.7 us)
+    if (W->type != HQ_TYPE_Q8_0 && K > 256 && sp.us < .85f * ws_us(W->type, M, N, K, nb, 1, wk.n_cu)) {
         *fused = 1;
         return hq_launch_gemm_sm(W, A, M, out, HQ_OUT_SWIGLU, 0, sp, nullptr, nullptr, st);
     }

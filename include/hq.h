@@ -113,8 +113,9 @@ int hq_gemv_swiglu(const hq_mat *gate, const hq_mat *up, const uint16_t *a, uint
 int hq_mat_upload_pair(const hq_wmat_t *gate, const hq_wmat_t *up, int device, hq_mat **out);
 /* out[M, rows] fp16 = silu(A . gate^T) * (A . up^T) for a pair matrix, A fp16 [M, K]; out 16-byte
  * aligned. Replaces gemm_w(gate) + gemm_w(up) + k_swiglu (src/cuda_backend.cu:845-849, :413-416):
- * for M > 64 the product never leaves the GEMM's tile (the epilogue of the full-K tile kernels
- * applies silu(g) * u), other shapes run one GEMM for both halves and a separate epilogue pass. */
+ * where one kernel holds the whole of K (M = 1, and larger M by estimated times) the product never
+ * leaves its tile, whose epilogue applies silu(g) * u; other shapes run one GEMM for both halves and
+ * a separate epilogue pass. */
 int hq_gemm_swiglu(const hq_mat *pair, const uint16_t *A, int M, uint16_t *out, void *stream);
 
 /* Option-row readout: out[b*k + j] = dot(H[b], head[ids[b*k + j]]) for b < B, j < k, fp32.

@@ -45,3 +45,18 @@ def test_small_tiles_keep(gtype, M, N, K):
     name = hq.gemm_kernel(gtype, M, N, K)
     assert name.startswith(("k_gemm_q8_0<", "k_gemm_q4_k<", "k_gemm_q6_k<", "k_gemm_kq<")) and not stream_k(gtype, M, N, K), name
     assert hq.gemm_workspace_bytes(gtype, M, N, K)[3]
+
+
+# hq_gemm_swiglu at M <= 64: (type, M, I, K, us of hq_gemm's kernel and the pass, us of one small-tile kernel)
+SWIGLU = [(Q8_0, 38, 832, 3328, 11.0, 18.8), (Q8_0, 3, 896, 3584, 9.2, 15.1), (Q8_0, 2, 2560, 2560, 9.6, 12.4), (Q8_0, 23, 3840, 3840, 15.1, 18.6),
+          (Q8_0, 17, 9728, 2560, 23.6, 25.9), (Q8_0, 16, 9728, 2560, 19.9, 17.3), (Q8_0, 2, 14336, 4096, 24.4, 23.7), (Q4_K, 16, 9728, 2560, 19.3, 16.4),
+          (Q4_K, 64, 9728, 2560, 34.3, 29.2), (Q4_K, 2, 5632, 2048, 14.4, 9.3), (Q5_K, 33, 1024, 512, 0, 0), (Q2_K, 64, 1024, 256, 0, 0)]
+
+
+@pytest.mark.parametrize("gtype,M,I,K,us,small_us", SWIGLU)
+def test_swiglu_route(gtype, M, I, K, us, small_us):
+    small = bool(hq.load().hq_internal_swiglu_small(gtype, M, I, K, 256))
+    if small_us > 1.04 * us:
+        assert not small
+    elif small_us <= .86 * us:  # (and the k-quants without a time, which all won)
+        assert small
