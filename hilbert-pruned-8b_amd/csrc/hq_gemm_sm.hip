@@ -418,6 +418,13 @@ __global__ void __launch_bounds__(SM_NT) k_gemm_kq(SmArgs g) {
     sm_tile<T, MB, KW>(g, lds);
 }
 
+// Workgroups of a launch: column tiles padded to whole turns over the XCDs; 0 where their threads would pass the 2^32 - 1
+// that a launch can have (outputs of some 50 GB: no plan then, another kernel runs)
+static unsigned sm_grid(long mt, long nt, long parts) {
+    const long n = (nt < 8 ? nt : 8 * ((nt + 7) / 8)) * mt * parts;
+    return n * SM_NT < 1l << 32 ? (unsigned)n : 0u;
+}
+
 hipError_t hq_launch_gemm_sm(const hq_dev_mat *W, const uint16_t *A, int M, void *C, int c_f32, int accumulate, const HqSmPlan &p,
                              float *partials, int *counters, hipStream_t st) {
     if (p.parts < 1 || p.parts > SM_PARTS || (p.parts > 1 && (!partials || !counters))) return hipErrorInvalidValue;
@@ -429,7 +436,8 @@ hipError_t hq_launch_gemm_sm(const hq_dev_mat *W, const uint16_t *A, int M, void
     const int bn = 16 * SM_W / p.kw;
     g.mt = (M + 16 * p.mb - 1) / (16 * p.mb), g.nt = (g.N + bn - 1) / bn, g.ntiles = g.mt * g.nt;
     g.parts = p.parts, g.partials = partials, g.counters = counters;
-    const unsigned grid = (unsigned)((g.nt < 8 ? g.nt : 8 * ((g.nt + 7) / 8)) * g.mt * g.parts);
+    const unsigned grid = sm_grid(g.mt, g.nt, g.parts);
+    if (!grid) return hipErrorInvalidValue;
 #define SM_LAUNCH(k) k<<<grid, SM_NT, 0, st>>>(g); break
 #define SM_CASE(mb, kw)                                                             \
     switch (W->type) {                                                              \
@@ -483,6 +491,7 @@ HqSmPlan hq_sm_plan(const hq_dev_mat *W, int M, int n_cu, int max_parts) {
         const long mt = (M + 16 * mb - 1) / (16 * mb);
         const float bytes = 1e-6f * (float)(16 * mb * 512 + cols * 16 * sm_pitch(type));
         for (int parts = 1; parts <= std::min(max_parts, SM_PARTS) && (parts == 1 || (2 * parts <= U && mt * nt * parts <= n_cu)); parts++) {
+            if (!sm_grid(mt, nt, parts)) break;  // (K split or not, the next is larger)
             const long wgs = mt * nt * parts, rounds = nt < 8 ? (wgs + n_cu - 1) / n_cu : ((nt + 7) / 8 * mt * parts + xcd - 1) / xcd;
             const float stages = (float)((U + parts - 1) / parts);
             const float t = f.base + q6 + std::max(f.round, decode > .1f ? 3.f : 0.f) * (float)(rounds - 1) + (float)rounds * stages * (f.stage + decode) +

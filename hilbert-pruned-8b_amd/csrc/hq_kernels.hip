@@ -1517,7 +1517,7 @@ float cfg_us(const hq_dev_mat *W, int M, const GemmCfg &c, int n_cu) {
 // (M = 512, N = 1024, K = 2560, where small tiles take 12 us instead of 28).
 bool sm_better(const hq_dev_mat *W, int M, const GemmCfg &c, const HqSmPlan &p, int n_cu) {
     const int type = W->type, N = (int)W->rows, K = (int)W->cols;
-    if (c.rbm || c.rb8 || c.wr || c.wr8 || c.bt || (type == HQ_TYPE_Q8_0 && (c.ws8_nb || K <= 256))) return false;
+    if (!p.parts || c.rbm || c.rb8 || c.wr || c.wr8 || c.bt || (type == HQ_TYPE_Q8_0 && (c.ws8_nb || K <= 256))) return false;
     if (c.wide && !c.ws_nb && (K <= 256 || N < 64 || (M > 256 && (long)N * K > 1l << 21))) return false;
     if ((c.ws_nb || c.ws8_nb) && K <= 256) return false;
     return p.us < (M > 64 ? .92f : .97f) * cfg_us(W, M, c, n_cu);
@@ -1670,7 +1670,7 @@ GemmCfg gemm_cfg(const hq_dev_mat *W, int M, int n_cu) {
         const int N = (int)W->rows, K = (int)W->cols;
         float us = 0.f;
         const int parts = wr8_split(M, N, K, n_cu, &us);
-        const float now = c.ws8_nb ? cfg_us(W, M, c, n_cu) : std::min(cfg_us(W, M, c, n_cu), hq_sm_plan(W, M, n_cu).us);
+        const float now = c.ws8_nb ? cfg_us(W, M, c, n_cu) : std::min(cfg_us(W, M, c, n_cu), hq_sm_plan(W, M, n_cu).us);  // (few tiles: there is a plan)
         const bool full = c.ws8_parts > 1 && 5L * M * N * c.ws8_parts >= 4L * n_cu * 128 * 32 * c.ws8_nb;
         if (parts > 1 && !full && (K >= 6144 ? us < now : M <= 128 && parts <= 3 && c.ws8_nb && us < 1.03f * now))
             c.wr8 = true, c.wr8_parts = parts;
@@ -1957,7 +1957,7 @@ hipError_t hq_launch_gemm_swiglu(const hq_dev_mat *W, const uint16_t *A, int M, 
     const int nb = hq_ws_choose(M, N, wk.n_cu, &eff);
     // against the LDS-decode tile kernels: where the estimates are 15 % apart (1.39x over the 480 calls measured that run
     // them; without a margin Q6_K at K = 512 .. 768 lost a tenth: M = 341, I = 1024 7.0 -> 7.7 us)
-    if (W->type != HQ_TYPE_Q8_0 && K > 256 && sp.us < .85f * ws_us(W->type, M, N, K, nb, 1, wk.n_cu)) {
+    if (sp.parts && W->type != HQ_TYPE_Q8_0 && K > 256 && sp.us < .85f * ws_us(W->type, M, N, K, nb, 1, wk.n_cu)) {
         *fused = 1;
         return hq_launch_gemm_sm(W, A, M, out, HQ_OUT_SWIGLU, 0, sp, nullptr, nullptr, st);
     }

@@ -60,3 +60,11 @@ def test_swiglu_route(gtype, M, I, K, us, small_us):
         assert not small
     elif small_us <= .86 * us:  # (and the k-quants without a time, which all won)
         assert small
+
+
+@pytest.mark.parametrize("M,N,K", [(7456384, 4096, 288), (5161984, 5000, 416), (818304, 30000, 1312), (828288, 30000, 2592), (8388608, 9000, 96)])
+def test_launches_stay_within_a_grid(M, N, K):
+    """The largest calls of a Q8_0 matrix with a ragged K: a launch has fewer than 2^32 threads, so the plan is not the
+    small-tile kernels' (768 threads per 64 x 64 or 128 x 128 tile) but the persistent one."""
+    assert hq.gemm_kernel(Q8_0, M, N, K) == "k_gemm_q8_0<8, 2>" and stream_k(Q8_0, M, N, K)
+    assert -(-M // 64) * -(-N // 64) * 768 >= 1 << 32 or -(-M // 128) * -(-N // 128) * 768 >= 1 << 32
