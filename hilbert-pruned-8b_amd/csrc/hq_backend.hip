@@ -50,8 +50,9 @@ namespace {
             return hq_internal_fail("HIP %s failed: %s (%s:%d)", #call, hipGetErrorString(e_), __FILE__, __LINE__); \
     } while (0)
 
-// tokens per layer-loop pass: of 2048 the row blocks of attention share the CUs (512 of 32 rows, longest first)
-// and each weight is decoded once. 4 layers of 512, 2048 tokens: 803 us in two passes of 1024, 590 in one.
+// most tokens per layer-loop pass (hq_internal_pass_tokens): of 2048 the row blocks of attention share the CUs (512 of
+// 32 rows, longest first) and each weight is decoded once. 4 layers of 512, 2048 tokens: 803 us in two passes of 1024,
+// 590 in one.
 constexpr int CHUNK = 2048;
 constexpr int MAX_IDS = 4096;  // readout ids per forward
 
@@ -479,6 +480,15 @@ int be_last_hidden(hq_ref_backend_t *bb, float *out) {
     return 0;
 }
 
+}  // namespace
+
+// 2048 tokens where their activations leave half of the free memory to the GEMMs' workspaces and the caller, else 1024
+extern "C" int hq_internal_pass_tokens(size_t max_seq, size_t bytes_per_token, size_t free_bytes) {
+    const size_t t = 2 * CHUNK * bytes_per_token <= free_bytes ? CHUNK : CHUNK / 2;
+    return (int)std::min(t, max_seq);
+}
+
+namespace {
 // Shapes the kernels support, checked before anything is uploaded.
 int check_model(const hq_ref_model_t *m, size_t max_seq) {
     const hq_ref_config_t &c = m->cfg;
@@ -553,16 +563,25 @@ int init(HipBackend *b, const hq_ref_model_t *m, size_t max_seq) {
         if (dalloc(b, (void **)&d.kc, max_seq * kvw * sizeof(float)) || dalloc(b, (void **)&d.vc, max_seq * kvw * sizeof(float)))
             return -1;
     }
-    const size_t CH = (size_t)(max_seq < (size_t)CHUNK ? max_seq : (size_t)CHUNK);
-    b->chunk = (int)CH;
+    // activations of a pass: k and v rows of their own only where some layer has three matrices, gate and up products
+    // only where some layer has them apart
     const size_t qw = (size_t)c.n_heads * hd * (c.attn_gate ? 2 : 1), ow = (size_t)c.n_heads * hd;
-    if (dalloc(b, (void **)&b->x, CH * H * 4) || dalloc(b, (void **)&b->qb, CH * (qw + 2 * kvw) * 4) ||
-        dalloc(b, (void **)&b->kb, CH * kvw * 4) || dalloc(b, (void **)&b->vb, CH * kvw * 4) ||
-        dalloc(b, (void **)&b->qr, CH * ow * 4) || dalloc(b, (void **)&b->gb, CH * I * 4) ||
-        dalloc(b, (void **)&b->ub, CH * I * 4) || dalloc(b, (void **)&b->hb, CH * H * 2) ||
-        dalloc(b, (void **)&b->ob, CH * ow * 2) || dalloc(b, (void **)&b->fb, CH * I * 2) ||
-        dalloc(b, (void **)&b->d_tok, CH * 4) || dalloc(b, (void **)&b->d_ids, MAX_IDS * 4))
-        return -1;
+    bool qkv_one = false, kv_apart = false, gu_apart = false;
+    for (const DevLayer &d : b->L) qkv_one |= d.qkv != nullptr, kv_apart |= !d.qkv, gu_apart |= !d.pair;
+    const struct {
+        void **p;
+        size_t bytes;  // per token
+    } bufs[] = {{(void **)&b->x, H * 4}, {(void **)&b->qb, (qw + (qkv_one ? 2 * kvw : 0)) * 4}, {(void **)&b->kb, kv_apart ? kvw * 4 : 0},
+                {(void **)&b->vb, kv_apart ? kvw * 4 : 0}, {(void **)&b->qr, ow * 4}, {(void **)&b->gb, gu_apart ? I * 4 : 0},
+                {(void **)&b->ub, gu_apart ? I * 4 : 0}, {(void **)&b->hb, H * 2}, {(void **)&b->ob, ow * 2}, {(void **)&b->fb, I * 2},
+                {(void **)&b->d_tok, 4}};
+    size_t per_token = 0, free_bytes = 0, total = 0;
+    for (auto &x : bufs) per_token += x.bytes;
+    BCK(hipMemGetInfo(&free_bytes, &total));
+    b->chunk = hq_internal_pass_tokens(max_seq, per_token, free_bytes);
+    for (auto &x : bufs)
+        if (x.bytes && dalloc(b, x.p, (size_t)b->chunk * x.bytes)) return -1;
+    if (dalloc(b, (void **)&b->d_ids, MAX_IDS * 4)) return -1;
     BCK(hipHostMalloc((void **)&b->h_out, (MAX_IDS + H) * sizeof(float), hipHostMallocDefault));
     BCK(hipDeviceGetAttribute(&b->n_cu, hipDeviceAttributeMultiprocessorCount, b->device));
     if (dalloc(b, (void **)&b->att_part, hq_attn_work_bytes((int)hd, b->n_cu)) ||

@@ -2,6 +2,7 @@
 #ifndef HQ_INTERNAL_H
 #define HQ_INTERNAL_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include "hq.h"
@@ -21,6 +22,9 @@ const char *hq_internal_supported_types(void);
 /* Whether hq_gemm_swiglu on M <= 64 rows of a pair matrix of 2 * rows rows is one small-tile kernel (else hq_gemm's kernel
  * and a pass over its product); no device is touched. */
 int hq_internal_swiglu_small(int ggml_type, int M, uint32_t rows, uint32_t K, int n_cu);
+
+/* Tokens of the backend's layer-loop pass, for activations of bytes_per_token. */
+int hq_internal_pass_tokens(size_t max_seq, size_t bytes_per_token, size_t free_bytes);
 
 /* The rows of n matrices of one type and width (Hugging Face order, one after the other) as one resident matrix. */
 int hq_internal_upload_cat(const hq_wmat_t *const *w, int n, int device, hq_mat **out);

@@ -532,13 +532,16 @@ class RefModelView:
     Q4_K block arrays, as the reference's model_load would fill it for a GGUF Llama model: q/k in
     llama.cpp storage order with perm_heads, every layer LAYER_FULL, RMSNorm offset 0. Keeps the
     arrays alive while the view exists. model["types"] may give other ggml types for the layer
-    matrices by name (e.g. {"gate": Q4_K, "up": Q6_K}, as Q4_K_M files mix them)."""
+    matrices by name (e.g. {"gate": Q4_K, "up": Q6_K}, as Q4_K_M files mix them); the config may set
+    norm_offset, qk_norm (layers then have q_norm and k_norm) and attn_gate (q then has the rows
+    [q_h | gate_h] of each head, in that order)."""
 
     def __init__(self, model, gtype=Q8_0):
         c = model["cfg"]
         self.keep = []
         H, I, V = c["hidden"], c["intermediate"], c["vocab"]
         qw, kvw = c["n_heads"] * c["head_dim"], c["n_kv_heads"] * c["head_dim"]
+        gated = bool(c.get("attn_gate"))
 
         types = model.get("types", {})
 
@@ -555,7 +558,8 @@ class RefModelView:
         cfg = RefConfig()
         for k in ("hidden", "n_layers", "intermediate", "vocab", "n_heads", "n_kv_heads", "head_dim", "rot_dim"):
             setattr(cfg, k, c[k])
-        cfg.arch, cfg.eps, cfg.rope_theta, cfg.norm_offset = 1, c["eps"], c["rope_theta"], 0.0
+        cfg.arch, cfg.eps, cfg.rope_theta, cfg.norm_offset = 1, c["eps"], c["rope_theta"], c.get("norm_offset", 0.0)
+        cfg.attn_gate, cfg.qk_norm = gated, bool(c.get("qk_norm"))
         cfg.n_full, cfg.n_linear = c["n_layers"], 0
         for li in range(c["n_layers"]):
             cfg.layer_type[li] = 1
@@ -564,9 +568,11 @@ class RefModelView:
             d = self.layers[li]
             d.type, d.slot = 1, li
             d.in_norm, d.post_norm = vec(L["in_norm"]), vec(L["post_norm"])
-            d.q = wm(L["q"], qw, H, c["n_heads"])
-            d.k = wm(L["k"], kvw, H, c["n_kv_heads"])
-            d.v, d.o = wm(L["v"], kvw, H), wm(L["o"], H, qw)
+            d.q = wm(L["q"], qw * (2 if gated else 1), H, 0 if gated else c["n_heads"], "q")
+            if cfg.qk_norm:
+                d.q_norm, d.k_norm = vec(L["q_norm"]), vec(L["k_norm"])
+            d.k = wm(L["k"], kvw, H, c["n_kv_heads"], "k")
+            d.v, d.o = wm(L["v"], kvw, H, name="v"), wm(L["o"], H, qw, name="o")
             d.gate, d.up = wm(L["gate"], I, H, name="gate"), wm(L["up"], I, H, name="up")
             d.down = wm(L["down"], H, I, name="down")
         self.m = RefModel()

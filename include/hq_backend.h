@@ -91,7 +91,10 @@ struct hq_ref_backend {
 /* cuda_backend_create (src/cuda_backend.cu:1003-1024): uploads the model to `device` (matrices with
  * hq_mat_upload, norm vectors and RoPE frequencies as fp32) and returns the vtable, reset to
  * position 0. forward is synchronous at return, as the reference's; prompts longer than one chunk
- * are processed in chunks with a KV cache of max_seq positions per layer. */
+ * are processed in chunks with a KV cache of max_seq positions per layer. A chunk is 2048 tokens (1024
+ * where 2048 tokens' activations would take over half of the free device memory); a token's activations
+ * take 6 hidden + 10 heads * head_dim + 8 kv_heads * head_dim + 2 ffn bytes (with the output gate 4
+ * heads * head_dim more; 8 ffn more where some layer's gate and up differ in type). */
 hq_ref_backend_t *hip_backend_create(const hq_ref_model_t *m, size_t max_seq, int device, bool keep_quantized);
 
 /* cuda_selftest (src/cuda_backend.cu:1392-1466), for this backend: every GEMM path of hq_gemm on
