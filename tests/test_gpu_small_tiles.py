@@ -1,9 +1,11 @@
 """The small-tile GEMM kernels (hq_gemm_sm.hip) at the edges of their tiles and of their K shares: 1 .. 3
-super-blocks, a Q8_0 K that ends inside one, rows around 16 / 32 / 64, columns around 64, one column tile
-and more than eight, a K split over workgroups, every output mode, against the oracle.
+super-blocks, a Q8_0 K that ends inside one, rows around 16 / 32 / 64 and several hundred to thousand, columns
+around 64, one column tile and more than eight, a K split over workgroups, every output mode, against the oracle.
+Each case states whether these kernels run it (SMALL names them; the workspace tells them from the Stream-K
+kernels of the same names); the others are their neighbours across the dispatch rule, one super-block mostly.
 
-Bars: those of the parity tests (rel-L2 1e-3, max-abs 1e-2), and for the types whose weights these kernels
-never round (all but Q8_0) fp32 outputs within 2^-18 |W| @ |a| of the float64 product: products are exact
+Bars: those of the parity tests (rel-L2 1e-3, max-abs 1e-2), and where these kernels or Stream-K run the types
+whose weights they never round (all but Q8_0) fp32 outputs within 2^-18 |W| @ |a| of the float64 product: products are exact
 in fp32, so what is left are fp32 sums of at most 256 terms per super-block in 32-term steps, the
 super-blocks' and parts' sums and one product with d each, under 32 roundings of 2^-24 per path.
 """
@@ -12,12 +14,21 @@ import pytest
 
 import synth
 from conftest import max_abs, rel_l2
+from test_gemm_routes import stream_k
 
 pytestmark = pytest.mark.gpu
 TYPES = [synth.Q8_0, synth.Q2_K, synth.Q3_K, synth.Q4_K, synth.Q5_K, synth.Q6_K]
 SMALL = ("k_gemm_q8_0<", "k_gemm_q4_k<", "k_gemm_q6_k<", "k_gemm_kq<")
 SHAPES = [(2, 16, 256), (16, 63, 512), (17, 65, 768), (32, 520, 256), (33, 100, 512), (64, 129, 2560), (65, 640, 512),
-          (130, 250, 768), (200, 64, 4096), (48, 1000, 256), (70, 96, 256), (12, 2560, 2560)]
+          (130, 250, 768), (200, 64, 4096), (48, 1000, 256), (70, 96, 256), (12, 2560, 2560),
+          (65, 640, 256), (15, 63, 2560), (301, 520, 1280), (700, 136, 768), (1024, 512, 512), (2048, 64, 4096)]
+
+
+def small(gtype, M, N, K):
+    """Whether a case is meant to be theirs."""
+    if K <= 256:
+        return gtype not in (synth.Q8_0, synth.Q4_K) and M > 64 and N > 96
+    return gtype != synth.Q8_0 or M > 32 or K > 2048
 
 
 def f64(oracle, blocks, t, N, K, a):
@@ -34,6 +45,7 @@ def test_small_tiles(hqlib, oracle, gtype, M, N, K):
     a = synth.activations_f16(synth.Rng(32 + M), M, K)
     name = hqlib.gemm_kernel(gtype, M, N, K)
     print(f"[gpu] small tiles {synth.TYPE_NAMES[gtype]} M={M} N={N} K={K} {name}", flush=True)
+    assert (name.startswith(SMALL) and not stream_k(gtype, M, N, K)) == small(gtype, M, N, K), name
     W = hqlib.Mat(blocks, gtype, N, K)
     got = hqlib.gemm_np(W, a)
     c0 = synth.activations_f16(synth.Rng(33), M, N)

@@ -1,10 +1,10 @@
 """The SwiGLU FFN input (src/cuda_backend.cu:845-849 gate + up + k_swiglu :413-416) as one GEMM over a
 gate/up pair matrix (hq_mat_upload_pair + hq_gemm_swiglu), through the C ABI, against the oracle's
 gate and up matmuls: silu(g) * u in float64, the GPU's fp16 output within half an ulp of |y| on top
-of the 1e-2 bar. M > 64 runs the fused epilogue of the full-K tile kernels (the product never
-leaves the tile: the register-decode kernels k_gemm_q4_k_wr / k_gemm_q4_k_wr160 / k_gemm_q8_0_wr where
-their 128 x 192 or 128 x 160 tiles fill the CUs, e.g. M = 512 at I = 9728, else the LDS-decode
-kernels); other M run one GEMM for both halves and a separate epilogue pass."""
+of the 1e-2 bar. Fused epilogues (the product never leaves the kernel): the GEMVs at M = 1, the small-tile
+kernels, and for M > 64 the register-decode kernels k_gemm_q4_k_wr / k_gemm_q4_k_wr160 / k_gemm_q8_0_wr where
+their 128 x 192 or 128 x 160 tiles fill the CUs, e.g. M = 512 at I = 9728, or the LDS-decode kernels; other
+shapes run one GEMM for both halves and a separate epilogue pass."""
 import numpy as np
 import pytest
 
