@@ -16,6 +16,10 @@
 //     four blocks, and a lane ends with 16 neighbouring dims of its row.
 // Row sums stay per lane until the end; the row maximum takes two lane exchanges per tile.
 //
+// Masked positions of a tile enter the output product with weight 0, not left out: an infinite or NaN value row of a
+// later token of the same pass makes NaN of earlier rows of its block. The pass's last row attends to every one of
+// them and is not finite either way.
+//
 // Bound: the fp32 matrix rate (256 FLOP per clock and CU); keys and values come from L2 straight into
 // the operand registers (16 QB rows per read), V a tile's score phase ahead, K a softmax and output
 // phase ahead. Measured (8 heads of 64, against one wave per token and head with vector dot products):

@@ -4,7 +4,7 @@
 // C[M,N] (+)= A[M,K] . W^T, A fp16, W GGUF blocks resident in HBM (block layouts: hq_kquant.h,
 // hq_q6k.hip, hq_kernels.hip; reference arithmetic cleanroom-transformer/src/ggml_quant.h:95-169).
 //
-// A workgroup of eight waves computes a tile of 16 MB rows x 16 CW columns over K, or over one of
+// A workgroup of eight consumer and four loader waves computes a tile of 16 MB rows x 16 CW columns over K, or over one of
 // `parts` ranges of it (tile_finish adds them). K runs in stages of one super-block (256 values) through
 // a ring of NST LDS slots: the tile's activations and its columns' super-blocks as they lie in HBM, all
 // by LDS DMA with neighbouring lanes on neighbouring bytes (the MFMA operand order, 16 rows by 64 bytes
@@ -15,7 +15,13 @@
 //
 // Why: a K loop inside one wave set leaves most CUs idle or a long serial chain where tiles are few, and
 // cutting K over workgroups costs a round trip through memory per tile; here a tile is small (N = 2560:
-// 80 of 32 columns) and its K still goes through 8 waves.
+// 40 of 64 columns) and its K still goes through 8 waves.
+//
+// What bounds it: the chain of stages, each a barrier, the decode (Q6_K at M = 37, N = 2560, K = 9728: 6.7 VALU
+// instructions per MFMA; Q4_K at M = 256, N = 1024, K = 2560: 10) and few products per decoded operand (2 or 4 row
+// blocks). There the matrix cores are busy 18 and 12 % of the cycles; for the first, HBM delivers 1.9 TB/s and L2 3.2,
+// both well below what they can. Against the Stream-K kernels: the first shape 27.0 -> 15.5 us, the second 26.1 -> 9, Q4_K M = 16,
+// N = K = 2560 11.1 -> 7.4.
 //
 // Operands of v_mfma_f32_16x16x32_f16 for k-step j of a half super-block: lane (ln, lg) holds row
 // (column) ln, values 32 j + 8 lg .. + 7. Weights are never rounded, except Q8_0's (fp16(q d), as in

@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr(Wr8Args g) { w8_tile<fal
 // tiles leave CUs idle, and the LDS-decode kernel's split (two waves' decode and its ring of 128-k stages) runs at
 // half this loop's rate. A 256-wide super-stage takes 1.6 us with few workgroups, 2.1 with 224 (L2); launches,
 // prologue, parts' round trip and sum 9 us + 0.23 us per MB of parts. M = 384, N = 4096, K = 15360: 96 -> 57 us
-// (839 TFLOP/s); M = 512, N = 2560, K = 9728: 37.5 -> 34 (750); M = 128: 26.3 -> 19.5 (327).
+// (839 TFLOP/s); M = 128, N = 2560, K = 9728: 26.3 -> 19.5 (327).
 __global__ void __launch_bounds__(W8_NT) k_gemm_q8_0_wr_ks(Wr8Args g) { w8_tile<true>(g); }
 }  // namespace
 

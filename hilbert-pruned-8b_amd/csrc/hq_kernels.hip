@@ -1513,8 +1513,8 @@ float cfg_us(const hq_dev_mat *W, int M, const GemmCfg &c, int n_cu) {
 // N = 4096, K = 96 3.9 -> 6.1.
 // Never for the register-decode kernels, the mid-M ones (as fast or faster where they apply: Q4_K M = 40, N = 7680,
 // K = 2048 10.4 against 11.7 us) and Q8_0's LDS-decode tiles, whose few losses would not pay for a rule. The wide Q4_K
-// kernel keeps K <= 256, N < 64 and M > 256 with over 2^21 weights whatever the estimates: its own tests lie there
-// (M = 512, N = 1024, K = 2560, where small tiles take 12 us instead of 28).
+// kernel keeps K <= 256, N < 64 and M > 256 with over 2^21 weights whatever the estimates, though small tiles are
+// often the faster there (M = 512, N = 1024, K = 2560: 12 us instead of 28): its own tests lie in that range.
 bool sm_better(const hq_dev_mat *W, int M, const GemmCfg &c, const HqSmPlan &p, int n_cu) {
     const int type = W->type, N = (int)W->rows, K = (int)W->cols;
     if (!p.parts || c.rbm || c.rb8 || c.wr || c.wr8 || c.bt || (type == HQ_TYPE_Q8_0 && (c.ws8_nb || K <= 256))) return false;
@@ -1663,9 +1663,10 @@ GemmCfg gemm_cfg(const hq_dev_mat *W, int M, int n_cu) {
     // 15360, M = 65 .. 1500: all faster, 1.04 to 2.2x). For a shorter K only over one row tile in 2 or 3 parts (M = 65,
     // N = 15360, K = 4096: 32.4 -> 24.0; M = 128, N = 19456, K = 2560: 25.9 -> 24.3): with more row tiles or parts
     // their sum takes what the split saves (M = 128, N = 9728, K = 2560: 16.6 against 17.9; M = 512, N = 2560,
-    // K = 4096: 21.7 against 21.4 at best). Not where the LDS-decode kernel's own split fills 80 % of the chip with rows
-    // and columns that exist, the shapes that tests hold it to, where least is to be had (M = 512, N = 2560,
-    // K = 9728: 37.5 against 34; M = 256: 25.9 against 23.1).
+    // K = 4096: 21.7 against 21.4 at best); there with 3 % of slack, which is within either
+    // estimate's error. Not where the LDS-decode kernel's own split fills 80 % of the chip with rows and
+    // columns that exist: tests hold that kernel to such shapes. The split would still be some 10 % faster there
+    // (M = 512, N = 2560, K = 9728: 37.5 against 34; M = 256: 25.9 against 23.1).
     if (!c.wr8 && W->type == HQ_TYPE_Q8_0 && M > 64 && hq_wr8_fits(W, M)) {
         const int N = (int)W->rows, K = (int)W->cols;
         float us = 0.f;
@@ -1904,9 +1905,10 @@ size_t hq_swiglu_sums_bytes(const hq_dev_mat *W, int M, int n_cu) {
 float pass_us(int M, int N) { return 2.2f + 2.6e-6f * (float)M * (float)N; }
 
 // M <= 64 of a pair matrix: the small-tile kernels with the epilogue in each tile (K in one workgroup) where their estimate
-// is below that of hq_gemm's kernel (less 8 % unless that is a small-tile one too) and a pass over its fp32 product. Over 6000 calls (every type, I = 64 .. 15360): 1.37x for
-// the k-quants, nearly all of them; Q8_0 half of its calls, 1.09x, where taking every one lost up to 1.7x to the mid-M
-// kernel's K split (M = 38, I = 832, K = 3328: 11.0 -> 18.8 us). Q8_0 of one super-block: 0.79 to 1.2x, so not.
+// is below that of hq_gemm's kernel (less 8 % unless that is a small-tile one too) and a pass over its fp32 product. Over
+// 6000 calls (every type, I = 64 .. 15360): 1.37x for the k-quants, nearly all of them; Q8_0 half of its calls, 1.09x,
+// where taking every one lost up to 1.7x to the mid-M kernel's K split (M = 38, I = 832, K = 3328: 11.0 -> 18.8 us).
+// Q8_0 of one super-block: 0.79 to 1.2x, so not.
 bool hq_swiglu_small(const hq_dev_mat *W, int M, int n_cu) {
     if (W->type == HQ_TYPE_Q8_0 && W->cols <= 256) return false;
     const GemmCfg c = gemm_cfg(W, M, n_cu);
